@@ -176,3 +176,35 @@ def test_device_cu_seqlens_make_no_host_read(pkg, dev, dtype):
     assert torch.equal(got, want)
     assert not got[:3].any() and not got[3456:].any()
     _check(got, q, k, v, cu, cu, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("h", [3, 200])  # blocks of 128 queries, and of 256
+def test_key_counts_at_step_and_block_edges(pkg, dev, dtype, d, h):
+    """Key counts around the 32-key steps and 64-key blocks of the 16-bit kernels, query counts
+    around their tiles.  The value row after every sequence's last key is infinite: no step may let
+    it in.  A last key whose own value is infinite gives that infinity, not NaN (zero times it)."""
+    rng = np.random.default_rng(100 * h + d)
+    lens = [1, 31, 32, 33, 63, 64, 65, 95, 97, 128, 129, 191, 193]
+    cu_kv, keep = [0], []
+    for n in lens:  # a gap row of infinities after each sequence belongs to an empty sequence's keys
+        cu_kv += [cu_kv[-1] + n, cu_kv[-1] + n + 1]
+        keep += [True, False]
+    nq = [1, 31, 33, 127, 129, 255, 257, 2, 32, 64, 128, 256, 5]
+    cu_q = [0]
+    for n in nq:
+        cu_q += [cu_q[-1] + n, cu_q[-1] + n]
+    q, k, v = _inputs(rng, cu_q[-1], cu_kv[-1], h, d, dtype)
+    gap = torch.tensor(cu_kv[1::2])
+    v[gap] = float("inf")
+    print(f"  attention key counts {dtype} D={d} H={h}", flush=True)
+    out = pkg.sparse_attention(q.to(dev), k.to(dev), v.to(dev), cu_q, cu_kv)
+    torch.cuda.synchronize()
+    v[gap] = 0
+    hs = [0, h - 1]  # heads are independent: two of them against the oracle
+    _check(out[:, hs], q[:, hs], k[:, hs], v[:, hs], cu_q, cu_kv, dtype)
+    last = torch.tensor(cu_kv[1::2]) - 1
+    v[last] = float("inf")
+    out = pkg.sparse_attention(q.to(dev), k.to(dev), v.to(dev), cu_q, cu_kv)
+    assert bool((out == float("inf")).all())
