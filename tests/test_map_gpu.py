@@ -108,6 +108,26 @@ def test_map_dense_and_sparse_extremes(pkg, dev, method):
         _build(pkg, dev, dup, 1, (64, 64, 64), method=method)
 
 
+@pytest.mark.parametrize("order", ["sorted", "reversed", "half_shuffled"])
+def test_map_near_sorted_input(pkg, dev, order):
+    """Rows (almost) in key order: a bucket's elements come as one or two long runs of a tile, which
+    a whole wave expands past 128 (127, 128 and 129 among them), in buckets of one chunk (4096
+    elements) and of several."""
+    rows = []
+    for x, n in enumerate((1, 127, 128, 129, 191, 4095, 4096, 4097, 9001, 200)):
+        k = np.arange(n)
+        rows.append(np.stack([np.zeros(n, int), np.full(n, x), k // 200, k % 200], axis=1))
+    coords = np.concatenate(rows).astype(np.int32)
+    if order == "reversed":
+        coords = coords[::-1]
+    elif order == "half_shuffled":
+        rng = np.random.default_rng(3)
+        some = rng.permutation(len(coords))[:len(coords) // 2]
+        coords[np.sort(some)] = coords[some]
+    m = _build(pkg, dev, coords, 1, (512, 512, 512), method="radix")
+    _check(m, coords, 1, (512, 512, 512), (1, 1, 1))
+
+
 @pytest.mark.parametrize("method", METHODS)
 def test_map_bucket_over_65536(pkg, dev, method):
     """A dense 256x512 half slice of 512^3 is one 2^17-cell key bucket of 131072 voxels: past the

@@ -27,8 +27,9 @@
 namespace tsc {
 namespace {
 
-constexpr int RT = 256;             // threads per block
-constexpr int RI = 16;              // items per thread
+constexpr int RT = 512;             // threads per block (256 x 16: the 1.5 M voxel map, whose
+                                    // largest bucket holds 8144, 113 us against 104)
+constexpr int RI = 8;               // items per thread
 constexpr int RTILE = RT * RI;      // elements per tile
 constexpr int WAVES = RT / 64;
 constexpr int TBMAX = 10;           // bucket digit bits
@@ -474,10 +475,10 @@ __global__ void __launch_bounds__(RT)
                        int32_t* __restrict__ col_start, GatherSrc<K> gs) {
   // smem: the key bitmap, or the LSD digit counters run[LNB] + wcnt[WAVES][LNB]; before either,
   // the gather pipeline's expanded source positions of the bucket's elements.
-  __shared__ __attribute__((aligned(16))) uint32_t smem[kBitmapWords];
+  __shared__ __attribute__((aligned(16))) uint32_t
+      smem[kBitmapWords > LNB * (WAVES + 1) ? kBitmapWords : LNB * (WAVES + 1)];
   __shared__ __attribute__((aligned(16))) uint16_t wpre[kBitmapWords];  // set bits before each word
   __shared__ int wsum[WAVES];
-  static_assert(kBitmapWords >= LNB * (WAVES + 1), "LSD counters alias the bitmap");
   uint32_t* bits = smem;
   int* run = (int*)smem;
   int(*wcnt)[LNB] = (int(*)[LNB])((int*)smem + LNB);
@@ -498,6 +499,7 @@ __global__ void __launch_bounds__(RT)
   // t*PTILE + ra[k].  The source positions of RTILE elements at a time are expanded into LDS
   // (pos[i]), so each element costs one LDS read.
   constexpr int kRunsPerThread = (kGatherTiles + RT - 1) / RT;
+  constexpr int kLongRun = 128;
   int* const pos = (int*)smem;  // [RTILE] expanded source positions, before the bitmap
   static_assert(RTILE <= kBitmapWords, "expanded positions fit the bitmap's words");
   int ra[kRunsPerThread], rl[kRunsPerThread], rb0[kRunsPerThread];
@@ -547,10 +549,22 @@ __global__ void __launch_bounds__(RT)
       const int c1 = min(size, c0 + RTILE);
 #pragma unroll
       for (int k = 0; k < kRunsPerThread; ++k) {
-        const int t = k * RT + tid;
-        if (t >= nt) continue;
-        const int lo = max(rb0[k], c0), hi = min(rb0[k] + rl[k], c1);
-        for (int e = lo; e < hi; ++e) pos[e - c0] = t * PTILE + ra[k] + (e - rb0[k]);
+        if (k * RT >= nt) continue;  // uniform
+        // A run longer than kLongRun is expanded by its whole wave, 64 positions at a time: where
+        // the input is close to sorted (the children of a subdivision) a bucket is one or two runs
+        // of thousands, which one thread walked alone (map of 1.4 M children in 512^3, this
+        // kernel: 164 us, now 30).  Shuffled input has runs of ~8, one thread each.
+        const int lo = max(rb0[k], c0), hi = min(rb0[k] + rl[k], c1);  // empty: lo >= hi
+        const int src = (k * RT + tid) * PTILE + ra[k] - rb0[k];
+        const bool longrun = hi - lo > kLongRun;
+        if (!longrun)
+          for (int e = lo; e < hi; ++e) pos[e - c0] = src + e;
+        for (uint64_t m = __ballot(longrun); m; m &= m - 1) {  // wave-uniform
+          const int l = __ffsll((unsigned long long)m) - 1;
+          const int wlo = __builtin_amdgcn_readlane(lo, l), whi = __builtin_amdgcn_readlane(hi, l);
+          const int wsrc = __builtin_amdgcn_readlane(src, l);
+          for (int e = wlo + (tid & 63); e < whi; e += 64) pos[e - c0] = wsrc + e;
+        }
       }
       __syncthreads();
       if (in_regs) {
