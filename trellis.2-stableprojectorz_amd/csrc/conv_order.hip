@@ -288,20 +288,14 @@ __global__ void __launch_bounds__(kOrdThreads)
 constexpr int kGrChunk = 4096;   // rows per chunk (and at most this many entries)
 constexpr int kGrThreads = 512;
 constexpr int kGrTile = 256;     // rows per tile of the 256-row conv kernels
-constexpr int kGrPerThread = kGrChunk / kGrThreads;  // rows, and entries at most, per thread
+// Sets of up to kFewRows rows (conv_order_few_launch): 1024-row chunks, so that a small set still
+// gives several blocks and each a quarter of the passes.
+constexpr int kGrFewChunk = 1024;
+constexpr int kGrFewThreads = 256;
 static_assert(kOrdTilesPerWin * kOrdTile % kGrChunk == 0, "chunks never straddle a window");
-static_assert(kGrChunk % kGrTile == 0, "chunks hold whole tiles");
-static_assert(kGrTile <= kGrThreads, "one thread per tile slot");
+static_assert(kGrTile <= kGrThreads && kGrTile <= kGrFewThreads, "one thread per tile slot");
 
-// Entry state: mask (26 bits) | next position in the chunk << 26 | rows left << 40.  Positions
-// and counts reach kGrChunk itself (a run that ends the chunk), so each field has 14 bits.
-static_assert(kGrChunk < (1 << 14), "14-bit position and count fields");
-__device__ __forceinline__ uint32_t gr_mask(uint64_t e) { return (uint32_t)(e & 0x3ffffffu); }
-__device__ __forceinline__ int gr_pos(uint64_t e) { return (int)((e >> 26) & 0x3fffu); }
-__device__ __forceinline__ int gr_left(uint64_t e) { return (int)(e >> 40); }
-__device__ __forceinline__ uint64_t gr_make(uint32_t mask, int pos, int left) {
-  return (uint64_t)mask | ((uint64_t)pos << 26) | ((uint64_t)left << 40);
-}
+constexpr uint32_t kSpent = 1u << 31;  // in an entry's mask: no rows left
 
 // Inclusive wave64 scans on DPP lane moves (row_shr inside each 16-lane row, then row_bcast:15
 // and row_bcast:31 across rows); lanes whose source is outside the row keep the identity.
@@ -345,67 +339,71 @@ __device__ __forceinline__ int gr_digit(const int32_t* head, int e) {
   return 255 - (rows < 255 ? rows : 255);
 }
 
-__global__ void __launch_bounds__(kGrThreads)
+template <int CHUNK, int T>
+__global__ void __launch_bounds__(T)
     ord_greedy_kernel(const uint32_t* __restrict__ keys, const int32_t* __restrict__ vals,
                       int64_t n, int32_t* __restrict__ order) {
-  __shared__ int32_t head[kGrChunk + 1];  // run starts; later the tile's segment marks
-  __shared__ int32_t idxa[kGrChunk];      // entry order (sort); later each output slot's source
-  __shared__ int32_t buf[8 * kGrThreads + kGrChunk];  // sort counters | entry order; later masks
-  __shared__ int wsum[kGrThreads / 64];
-  __shared__ int wmax[kGrThreads / 64];
-  __shared__ int wtot[2][kGrThreads / 64];        // per-pass wave sums (two buffers by parity)
-  __shared__ uint32_t wbest[2][kGrThreads / 64];  // per-pass wave minima
-  __shared__ uint32_t wseed[kGrThreads / 64];
+  constexpr int P = CHUNK / T;  // rows, and entries at most, per thread
+  static_assert(CHUNK % kGrTile == 0, "chunks hold whole tiles");
+  static_assert(CHUNK <= (1 << 14), "14-bit entry indices in the growth candidates");
+  __shared__ int32_t head[CHUNK + 1];  // run starts; later the tile's segment marks
+  __shared__ int32_t idxa[CHUNK];      // entry order (sort); later each output slot's source
+  __shared__ int32_t buf[8 * T + CHUNK];  // sort counters | entry order; later masks
+  __shared__ int wsum[T / 64];
+  __shared__ int wmax[T / 64];
+  __shared__ int wtot[2][T / 64];        // per-pass wave sums (two buffers by parity)
+  __shared__ uint32_t wbest[2][T / 64];  // per-pass wave minima
+  __shared__ uint32_t wseed[T / 64];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int64_t c0 = (int64_t)blockIdx.x * kGrChunk;
-  const int nc = (int)(n - c0 < kGrChunk ? n - c0 : kGrChunk);
+  const int64_t c0 = (int64_t)blockIdx.x * CHUNK;
+  const int nc = (int)(n - c0 < CHUNK ? n - c0 : CHUNK);
 
   // Runs of equal keys: thread t owns positions [t*P, t*P + P).
   int nd;
   {
     uint32_t hb = 0;  // bit j: position p0 + j starts a run
-    const int p0 = tid * kGrPerThread;
+    const int p0 = tid * P;
     uint32_t prev = p0 > 0 && p0 <= nc ? keys[c0 + p0 - 1] : 0u;
 #pragma unroll
-    for (int j = 0; j < kGrPerThread; ++j) {
+    for (int j = 0; j < P; ++j) {
       const int i = p0 + j;
       const uint32_t k = i < nc ? keys[c0 + i] : 0u;
       hb |= (i < nc && (i == 0 || k != prev) ? 1u : 0u) << j;
       prev = k;
     }
-    int e = block_excl_scan(__popc(hb), wsum, kGrThreads / 64);
+    int e = block_excl_scan(__popc(hb), wsum, T / 64);
     nd = 0;
 #pragma unroll
-    for (int ww = 0; ww < kGrThreads / 64; ++ww) nd += wsum[ww];
+    for (int ww = 0; ww < T / 64; ++ww) nd += wsum[ww];
     for (uint32_t m = hb; m; m &= m - 1) head[e++] = p0 + __ffs(m) - 1;
     if (tid == 0) head[nd] = nc;
   }
   // Entries per thread: contiguous runs [ebeg, ebeg + ne).
-  const int E = (nd + kGrThreads - 1) / kGrThreads;
+  const int E = (nd + T - 1) / T;
   const int ebeg = tid * E;
   const int ne = max(0, min(nd - ebeg, E));
-  for (int i = tid; i < nd; i += kGrThreads) idxa[i] = i;
+  for (int i = tid; i < nd; i += T) idxa[i] = i;
   __syncthreads();
   // Stable LSD counting sort of the entries by gr_digit, three passes of 3 bits: per-thread digit
-  // counts in a digit-major [8][kGrThreads] matrix, one block scan, stable placement; the passes
+  // counts in a digit-major [8][T] matrix, one block scan, stable placement; the passes
   // alternate between idxa and idxb and end in idxb.
-  constexpr int kDig = 8, kCpt = kDig * kGrThreads / kGrThreads;  // counters per thread in the scan
-  int32_t* const cnt = buf;  // [kDig][kGrThreads]
-  int32_t* const idxb = buf + kDig * kGrThreads;
-  static_assert(kDig == 8 && kGrChunk <= kDig * kGrThreads, "counters, order and masks fit buf");
+  constexpr int kDig = 8, kCpt = kDig * T / T;  // counters per thread in the scan
+  int32_t* const cnt = buf;  // [kDig][T]
+  int32_t* const idxb = buf + kDig * T;
+  static_assert(kDig == 8 && CHUNK <= kDig * T, "counters, order and masks fit buf");
   for (int pass = 0; pass < 3; ++pass) {
     const int32_t* src = (pass & 1) ? idxb : idxa;
     int32_t* dst = (pass & 1) ? idxa : idxb;
     const int sh = 3 * pass;
     // column tid of the counter matrix belongs to this thread alone
-    for (int d = 0; d < kDig; ++d) cnt[d * kGrThreads + tid] = 0;
+    for (int d = 0; d < kDig; ++d) cnt[d * T + tid] = 0;
     for (int j = 0; j < ne; ++j)
-      ++cnt[((gr_digit(head, src[ebeg + j]) >> sh) & (kDig - 1)) * kGrThreads + tid];
+      ++cnt[((gr_digit(head, src[ebeg + j]) >> sh) & (kDig - 1)) * T + tid];
     __syncthreads();
     // exclusive scan of the counters in digit-major order: thread t scans [t*kCpt, t*kCpt + kCpt)
     int sum = 0;
     for (int q = 0; q < kCpt; ++q) sum += cnt[tid * kCpt + q];
-    int pre = block_excl_scan(sum, wsum, kGrThreads / 64);
+    int pre = block_excl_scan(sum, wsum, T / 64);
     for (int q = 0; q < kCpt; ++q) {
       const int c = cnt[tid * kCpt + q];
       cnt[tid * kCpt + q] = pre;
@@ -414,27 +412,32 @@ __global__ void __launch_bounds__(kGrThreads)
     __syncthreads();
     for (int j = 0; j < ne; ++j) {
       const int e = src[ebeg + j];
-      dst[cnt[((gr_digit(head, e) >> sh) & (kDig - 1)) * kGrThreads + tid]++] = e;
+      dst[cnt[((gr_digit(head, e) >> sh) & (kDig - 1)) * T + tid]++] = e;
     }
     __syncthreads();
   }
-  // This thread's entries (sorted positions ebeg..ebeg+ne) into registers; masks to LDS.
-  uint64_t my[kGrPerThread];
+  // This thread's entries (sorted positions ebeg..ebeg+ne) into registers: mask (with kSpent set
+  // once no row is left), next position in the chunk, rows left; masks to LDS.
+  uint32_t em[P];
+  int pos[P], left[P];
 #pragma unroll
-  for (int j = 0; j < kGrPerThread; ++j) {
-    my[j] = 0;
+  for (int j = 0; j < P; ++j) {
+    em[j] = kSpent;
+    pos[j] = left[j] = 0;
     if (j < ne) {
       const int e = idxb[ebeg + j];
       const int a = head[e];
       const uint32_t rank = keys[c0 + a];
-      my[j] = gr_make(rank ^ (rank >> 1), a, head[e + 1] - a);
+      em[j] = rank ^ (rank >> 1);
+      pos[j] = a;
+      left[j] = head[e + 1] - a;
     }
   }
   __syncthreads();
   uint32_t* const emask = (uint32_t*)buf;
 #pragma unroll
-  for (int j = 0; j < kGrPerThread; ++j)
-    if (j < ne) emask[ebeg + j] = gr_mask(my[j]);
+  for (int j = 0; j < P; ++j)
+    if (j < ne) emask[ebeg + j] = em[j];
   // Segment marks over the chunk's output slots (the run starts are no longer needed): a taking
   // entry marks the first slot it fills with (its source position - that slot + kMarkOff); the
   // slots after it up to the next mark come from the same run.  The marks are resolved once for
@@ -444,7 +447,7 @@ __global__ void __launch_bounds__(kGrThreads)
   // the first mark.
   int32_t* const mark = head;
   constexpr int kMarkOff = 1 << 16;
-  for (int i = tid; i < nc; i += kGrThreads) mark[i] = 0;
+  for (int i = tid; i < nc; i += T) mark[i] = 0;
   const int ntile = (nc + kGrTile - 1) / kGrTile;
   for (int t = 0; t < ntile; ++t) {
     const int rows = min(kGrTile, nc - t * kGrTile);
@@ -452,34 +455,37 @@ __global__ void __launch_bounds__(kGrThreads)
     // seed: the first entry with rows left
     uint32_t fa = ~0u;
 #pragma unroll
-    for (int j = 0; j < kGrPerThread; ++j) {
+    for (int j = 0; j < P; ++j) {
       if (j >= E) break;  // uniform: no thread owns more entries
-      if (j < ne && gr_left(my[j]) > 0 && fa == ~0u) fa = (uint32_t)(ebeg + j);
+      if (!(em[j] & kSpent) && fa == ~0u) fa = (uint32_t)(ebeg + j);
     }
     fa = wave_incl_umin(fa);
     if (lane == 63) wseed[wid] = fa;
     __syncthreads();
 #pragma unroll
-    for (int ww = 0; ww < kGrThreads / 64; ++ww) fa = umin32(fa, wseed[ww]);
+    for (int ww = 0; ww < T / 64; ++ww) fa = umin32(fa, wseed[ww]);
     uint32_t orm = emask[fa];  // rows remain, so an entry with rows exists
     int need = rows, fill = 0;
     for (int iter = 0;; ++iter) {
-      if (iter >= 27) orm = ~0u;  // 26 growths fill OR; guard only
+      if (iter >= 27) orm = ~kSpent;  // 26 growths fill OR; guard only
       // One block reduction per pass: the rows of the entries inside OR (to be taken, in entry
       // order) and, among the other entries with rows left, the one whose mask adds the fewest
       // taps (lowest index on ties) -- the growth if the tile is still short.  Taking touches
-      // only entries inside OR, so the growth candidate stays valid after it.
+      // only entries inside OR, so the growth candidate stays valid after it.  A spent entry is
+      // never inside (kSpent is outside every OR), and its candidate keeps kSpent: it loses to
+      // any other.
       int sum = 0;
       uint32_t cand = ~0u;
+      uint32_t inside = 0u;  // bit j: entry j lies inside OR and has rows left
 #pragma unroll
-      for (int j = 0; j < kGrPerThread; ++j) {
+      for (int j = 0; j < P; ++j) {
         if (j >= E) break;
-        const int left = gr_left(my[j]);
-        if (j < ne && left > 0) {
-          const uint32_t out = gr_mask(my[j]) & ~orm;
-          if (out == 0u) sum += left;
-          else cand = umin32(cand, ((uint32_t)__popc(out) << 14) | (uint32_t)(ebeg + j));
-        }
+        const uint32_t out = em[j] & ~orm;
+        const uint32_t c =
+            ((uint32_t)__popc(out) << 14) | (uint32_t)(ebeg + j) | (out & kSpent);
+        sum += out == 0u ? left[j] : 0;
+        inside |= out == 0u ? 1u << j : 0u;
+        cand = umin32(cand, out == 0u ? ~0u : c);
       }
       const int incl = wave_incl_add(sum);
       const uint32_t wmin = wave_incl_umin(cand);
@@ -493,39 +499,39 @@ __global__ void __launch_bounds__(kGrThreads)
       int o = incl - sum, tot = 0;
       uint32_t best = ~0u;
 #pragma unroll
-      for (int ww = 0; ww < kGrThreads / 64; ++ww) {
+      for (int ww = 0; ww < T / 64; ++ww) {
         const int v = wt[ww];
         tot += v;
         o += ww < wid ? v : 0;
         best = umin32(best, wb[ww]);
       }
 #pragma unroll
-      for (int j = 0; j < kGrPerThread; ++j) {
+      for (int j = 0; j < P; ++j) {
         if (j >= E) break;
-        const int left = gr_left(my[j]);
-        if (j < ne && left > 0 && (gr_mask(my[j]) & ~orm) == 0u && o < need) {
-          const int take = min(left, need - o);
-          const int pos = gr_pos(my[j]);
-          mark[base + fill + o] = pos - (base + fill + o) + kMarkOff;
-          my[j] = gr_make(gr_mask(my[j]), pos + take, left - take);
-          o += left;
+        if ((inside >> j & 1u) && o < need) {
+          const int take = min(left[j], need - o);
+          mark[base + fill + o] = pos[j] - (base + fill + o) + kMarkOff;
+          o += left[j];
+          pos[j] += take;
+          left[j] -= take;
+          if (left[j] == 0) em[j] |= kSpent;
         }
       }
       const int got = min(tot, need);
       fill += got;
       need -= got;
       if (need == 0) break;
-      orm |= best != ~0u ? emask[best & 0x3fffu] : ~0u;
+      orm |= best < kSpent ? emask[best & 0x3fffu] : ~kSpent;
     }
   }
   __syncthreads();  // marks of every thread
   // Slot r takes its source from the last mark at or before r: thread t scans its slots
   // [t*P, t*P + P), the last mark before them is an exclusive max scan over the threads.
-  const int r0 = tid * kGrPerThread;
-  int lastj[kGrPerThread];
+  const int r0 = tid * P;
+  int lastj[P];
   int last = -1;
 #pragma unroll
-  for (int j = 0; j < kGrPerThread; ++j) {
+  for (int j = 0; j < P; ++j) {
     if (r0 + j < nc && mark[r0 + j] != 0) last = r0 + j;
     lastj[j] = last;
   }
@@ -536,7 +542,7 @@ __global__ void __launch_bounds__(kGrThreads)
   if (lane == 0) before = -1;
   for (int ww = 0; ww < wid; ++ww) before = max(before, wmax[ww]);
 #pragma unroll
-  for (int j = 0; j < kGrPerThread; ++j) {
+  for (int j = 0; j < P; ++j) {
     const int r = r0 + j;
     if (r < nc) {
       const int l = lastj[j] >= 0 ? lastj[j] : before;
@@ -583,8 +589,8 @@ int conv_order_launch(tsc_ctx* ctx, const int32_t* nbr, const int32_t* perm, int
     std::swap(kc, kn);
     std::swap(vc, vn);
   }
-  ord_greedy_kernel<<<(unsigned)((N + kGrChunk - 1) / kGrChunk), kGrThreads, 0, s>>>(kc, vc, N,
-                                                                                     order);
+  ord_greedy_kernel<kGrChunk, kGrThreads>
+      <<<(unsigned)((N + kGrChunk - 1) / kGrChunk), kGrThreads, 0, s>>>(kc, vc, N, order);
   return check_hip(hipGetLastError(), "conv_order launch");
 }
 
