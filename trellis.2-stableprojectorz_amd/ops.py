@@ -160,9 +160,25 @@ def build_neighbor_map(coords: torch.Tensor, spatial_shape, batch_size: int,
     return nmap
 
 
-def _nbr_and_order(nmap, order):
+def _key_order_will_do(n: int, ci: int, co: int, elem: int) -> bool:
+    """Whether a conv is as fast in key order as in the conv order, so that none need be built.
+
+    The conv order saves taps of most row tiles, but some tile still has nearly all 27; while every
+    tile of the generic kernel (64 rows x 64 columns; row sizes or Co that are not multiples of 32)
+    has a CU of its own, that tile sets the time.  8->64 bf16 on 6007 voxels: 14.5 us either way,
+    and building the order takes 140 us; 40->72 fp32: 62 us either way (188 tiles), but 65 in the
+    conv order against 77 on 9001 (282 tiles, past the 256 CUs).  The tuned kernels, whose waves
+    keep more loads in flight, lose 1-4 % in key order at any size: they keep the conv order."""
+    generic = (ci * elem) % 32 != 0 or co % 32 != 0
+    return generic and -(-n // 64) * -(-co // 64) <= 256
+
+
+def _nbr_and_order(nmap, order, key_order: bool = False):
+    """Neighbor table and row order; key_order: the map's key order will do if no other is there."""
     if isinstance(nmap, NeighborMap):
-        return nmap.nbr, (nmap.conv_order() if order is None else order)
+        if order is None:
+            order = nmap.perm if key_order and nmap._conv_order is None else nmap.conv_order()
+        return nmap.nbr, order
     return nmap, order
 
 
@@ -181,10 +197,13 @@ def sparse_conv3d(feats: torch.Tensor, weight: torch.Tensor, bias, nmap, order=N
 
     weight is (Co,Kd,Kh,Kw,Ci) = (Co,3,3,3,Ci), same dtype as feats; accumulation is fp32.
     nmap is a NeighborMap (its cached row order, or for Ci = 32 in fp16/bf16 its cached gather
-    plan, is used for locality) or an (N,27) int32 table.
+    plan, or for small convs of the generic kernel its key order, is used for locality) or an (N,27) int32 table.
     """
     plan = nmap.gather_plan() if _uses_gather_plan(nmap, order, feats, weight) else None
-    nbr, order = (nmap.nbr, None) if plan is not None else _nbr_and_order(nmap, order)
+    key_order = (feats.dim() == 2 and weight.dim() == 5 and
+                 _key_order_will_do(feats.shape[0], weight.shape[4], weight.shape[0],
+                                    feats.element_size()))
+    nbr, order = (nmap.nbr, None) if plan is not None else _nbr_and_order(nmap, order, key_order)
     if weight.dim() != 5 or tuple(weight.shape[1:4]) != (3, 3, 3):
         raise TscError(_lib.TSC_ERR_UNSUPPORTED, f"weight must be (Co,3,3,3,Ci), got {tuple(weight.shape)}")
     co, ci = weight.shape[0], weight.shape[4]
