@@ -247,6 +247,11 @@ int tsc_linear(tsc_ctx* ctx, int32_t dtype, const void* x, int64_t N, int32_t Ci
  * where the TS port only doubles the spatial shape); the spatial shape and the scale of the
  * result are twice the input's. */
 int tsc_subdivide_count(tsc_ctx* ctx, const uint8_t* keep, int64_t N, int64_t* count);
+/* The same count, and with it the batch index of the last kept child's parent (-1: none kept) --
+ * one read-back for both, so that a caller needs no second one for the children's batch size.
+ * coords: the (N,4) parents. */
+int tsc_subdivide_count_batch(tsc_ctx* ctx, const int32_t* coords, const uint8_t* keep, int64_t N,
+                              int64_t* count, int32_t* last_batch);
 int tsc_subdivide(tsc_ctx* ctx, const int32_t* coords, int64_t N, int32_t dtype, const void* feats,
                   int32_t C, const uint8_t* keep, int32_t* coords_out, void* feats_out);
 

@@ -77,6 +77,27 @@ def test_subdivide_rejects_bad_arguments(pkg, dev):
         pkg.sparse_subdivide(c, None, torch.zeros(4, dtype=torch.int32, device=dev))
 
 
+@pytest.mark.parametrize("n,last", [(1, 0), (255, 254), (256, 0), (257, 256), (257, 255),
+                                    (300000, 299999), (300000, 7), (5, None)])
+def test_subdivide_batch_size(pkg, dev, n, last):
+    """The children's batch size is the batch of the last parent with a kept child + 1, wherever it
+    lies in its 256-parent tile and in the scan's 1024-tile rounds; without children it is 1."""
+    coords = torch.zeros((n, 4), dtype=torch.int32)
+    coords[:, 0] = torch.arange(n) // 3
+    coords[:, 1] = torch.arange(n) % 3
+    keep = torch.zeros(n, dtype=torch.uint8)
+    if last is not None:
+        keep[::5] = 0x81
+        keep[last + 1:] = 0
+        keep[last] = 0x10
+    x = pkg.SparseTensor(torch.zeros((n, 2), device=dev), coords.to(dev), spatial_shape=[3, 1, 1],
+                         batch_size=n // 3 + 1)
+    y = pkg.SparseSubdivide()(x, keep.to(dev))
+    assert y.coords.shape[0] == int(sum(bin(b).count("1") for b in keep.tolist()))
+    assert y.batch_size == (1 if last is None else last // 3 + 1)
+    assert y.batch_size == len(pkg.sparse_tensor.compute_layout(y.coords))
+
+
 def test_subdivide_module_then_conv(pkg, dev):
     """SparseSubdivide output: doubled shape and scale, and a conv on it uses the children's own
     neighbor map (bit-exact against the oracle's map of the children)."""

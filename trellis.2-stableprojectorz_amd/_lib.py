@@ -77,6 +77,8 @@ _SIGNATURES = {
     "tsc_resblock": (_I32, [_P, _I32, _P, _P, _P, _I64, _I32, _P, _P, _P, _P, _F32, _P, _P, _P]),
     "tsc_linear": (_I32, [_P, _I32, _P, _I64, _I32, _P, _P, _P, _I32, _P]),
     "tsc_subdivide_count": (_I32, [_P, _P, _I64, ctypes.POINTER(_I64)]),
+    "tsc_subdivide_count_batch": (_I32, [_P, _P, _P, _I64, ctypes.POINTER(_I64),
+                                         ctypes.POINTER(_I32)]),
     "tsc_subdivide": (_I32, [_P, _P, _I64, _I32, _P, _I32, _P, _P, _P]),
     "tsc_attention": (_I32, [_P, _I32, _P, _P, _P, _P, _P, _I32, _I64, _I64, _I32, _I32, _F32,
                              _I32, _P]),

@@ -603,7 +603,20 @@ int tsc_subdivide_count(tsc_ctx* ctx, const uint8_t* keep, int64_t N, int64_t* c
   if (N < 0 || !count) return fail(TSC_ERR_INVALID, "subdivide_count: bad arguments");
   if (N > 0 && !keep) return fail(TSC_ERR_INVALID, "subdivide_count: null keep mask");
   DeviceGuard g(ctx->device);
-  return subdivide_count_launch(ctx, keep, N, count);
+  return subdivide_count_launch(ctx, keep, N, nullptr, count, nullptr);
+}
+
+int tsc_subdivide_count_batch(tsc_ctx* ctx, const int32_t* coords, const uint8_t* keep, int64_t N,
+                              int64_t* count, int32_t* last_batch) {
+  g_err[0] = 0;
+  int st = check_ctx(ctx);
+  if (st) return st;
+  if (N < 0 || !count || !last_batch)
+    return fail(TSC_ERR_INVALID, "subdivide_count_batch: bad arguments");
+  if (N > 0 && (!keep || !coords))
+    return fail(TSC_ERR_INVALID, "subdivide_count_batch: null coords / keep mask");
+  DeviceGuard g(ctx->device);
+  return subdivide_count_launch(ctx, keep, N, coords, count, last_batch);
 }
 
 int tsc_subdivide(tsc_ctx* ctx, const int32_t* coords, int64_t N, int32_t dtype, const void* feats,

@@ -200,7 +200,8 @@ bool conv_gather_supported(const ConvArgs& a);
 int conv_gather_launch(tsc_ctx* ctx, const ConvArgs& a);
 
 // ---- launchers implemented in subdivide.hip ----
-int subdivide_count_launch(tsc_ctx* ctx, const uint8_t* keep, int64_t N, int64_t* count_host);
+int subdivide_count_launch(tsc_ctx* ctx, const uint8_t* keep, int64_t N, const int32_t* coords,
+                           int64_t* count_host, int32_t* last_batch);
 int subdivide_launch(tsc_ctx* ctx, const int32_t* coords, int64_t N, const void* feats,
                      int64_t row_bytes, const uint8_t* keep, int32_t* coords_out,
                      void* feats_out);

@@ -307,6 +307,13 @@ def sparse_subdivide(coords: torch.Tensor, feats: torch.Tensor | None = None,
     each with a copy of the parent's feature row; keep (uint8 (N,), bit c = keep child c) selects
     children (M = its set bits; counting them costs one stream sync), else M = 8N.
     """
+    return subdivide_with_batch(coords, feats, keep)[:2]
+
+
+def subdivide_with_batch(coords, feats=None, keep=None):
+    """sparse_subdivide, and the children's batch size (last row's batch index + 1, as
+    compute_layout) where the keep mask's count is read back anyway; None without a mask or without
+    children."""
     if coords.dtype != torch.int32 or coords.dim() != 2 or coords.shape[1] != 4:
         raise TscError(_lib.TSC_ERR_INVALID, "coords must be int32 of shape (N,4)")
     if feats is not None and (feats.dim() != 2 or feats.shape[0] != coords.shape[0]):
@@ -316,7 +323,13 @@ def sparse_subdivide(coords: torch.Tensor, feats: torch.Tensor | None = None,
     dev = _dev(coords, feats, keep)
     ctx = _lib.context(dev)
     n = coords.shape[0]
-    m = 8 * n if keep is None else subdivide_count(keep)
+    m, batch = 8 * n, None
+    if keep is not None:
+        count, last = ctypes.c_int64(0), ctypes.c_int32(-1)
+        check(ctx.lib.tsc_subdivide_count_batch(ctx.bind(), _p(coords), _p(keep), n,
+                                                ctypes.byref(count), ctypes.byref(last)))
+        m = int(count.value)
+        batch = last.value + 1 if last.value >= 0 else None
     coords_out = torch.empty((m, 4), dtype=torch.int32, device=coords.device)
     feats_out = None
     dtype, c = 0, 0
@@ -326,7 +339,7 @@ def sparse_subdivide(coords: torch.Tensor, feats: torch.Tensor | None = None,
     if m:
         check(ctx.lib.tsc_subdivide(ctx.bind(), _p(coords), n, dtype, _p(feats), c, _p(keep),
                                     _p(coords_out), _p(feats_out)))
-    return coords_out, feats_out
+    return coords_out, feats_out, batch
 
 
 def sparse_linear(x: torch.Tensor, weight: torch.Tensor, bias=None, residual=None,

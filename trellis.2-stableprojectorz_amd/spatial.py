@@ -28,9 +28,10 @@ def _double(f: Fraction) -> Fraction:
 
 class SparseSubdivide:
     def forward(self, x: SparseTensor, keep: torch.Tensor | None = None) -> SparseTensor:
-        coords, feats = ops.sparse_subdivide(x.coords, x.feats, keep)
+        coords, feats, batch = ops.subdivide_with_batch(x.coords, x.feats, keep)
         scale = Scale(_double(x.scale.x), _double(x.scale.y), _double(x.scale.z))
-        out = SparseTensor(feats, coords, scale=scale, cache=x._spatial_cache)
+        out = SparseTensor(feats, coords, scale=scale, cache=x._spatial_cache,
+                           batch_size=batch)
         out.register_spatial_cache("shape", [2 * s for s in x.spatial_shape])
         return out
 
