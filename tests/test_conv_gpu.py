@@ -439,3 +439,79 @@ def test_conv_rejects_invalid(pkg, dev):
     st = lib.lib.tsc_conv(lib.bind(), pkg._lib.TSC_F16, raw.data_ptr() + 1, w.data_ptr(), None,
                           m.nbr.data_ptr(), None, 1, 32, 48, raw.data_ptr() + 2)
     assert st == pkg._lib.TSC_ERR_INVALID
+
+
+def _random_table(n, seed, present=0.5):
+    """(n,27) neighbor table of random rows, tap 13 the row itself."""
+    rng = np.random.default_rng(seed)
+    nbr = rng.integers(0, n, (n, 27)).astype(np.int32)
+    nbr[rng.random((n, 27)) > present] = -1
+    nbr[:, 13] = np.arange(n)
+    return nbr
+
+
+def _conv64(f, w, b, nbr):
+    """fp64 conv on the tensors' device."""
+    out = b.double().expand(f.shape[0], -1).clone()
+    for v in range(27):
+        rows = torch.nonzero(nbr[:, v] >= 0).flatten()
+        wt = w[:, v // 9, v // 3 % 3, v % 3].double().t().contiguous()
+        out[rows] += f[nbr[rows, v].long()].double() @ wt
+    return out
+
+
+@pytest.mark.parametrize("n,ci,co", [
+    (1, 32, 64), (31, 48, 64), (65, 64, 64), (3000, 64, 128),        # 64 x 32 tiles
+    (16385, 48, 64), (20001, 32, 64),                                # 64 x 64
+    (32641, 32, 64), (33000, 80, 64), (40003, 64, 128),              # 128 x 64
+    (1, 32, 32 * 3), (127, 64, 32), (129, 48, 96), (5000, 128, 32)]) # 128 x 32
+def test_conv_fp32_split_tiles(pkg, dev, n, ci, co):
+    """fp32 convs on bf16 pieces, at the edges of every tile and with odd chunk counts per tap.  At
+    most 27 Ci products are summed in fp32, each sum rounding by at most 2^-24 of its size: 4e-6
+    of the result (2-norm) is some ten times the random walk of these roundings.  The same bits
+    from the noalloc entry, which splits the weights in the kernel, and in place on the residual."""
+    print(f"  conv fp32 split N={n} {ci}->{co}", flush=True)
+    nbr = torch.from_numpy(_random_table(n, n)).to(dev)
+    f = torch.from_numpy(pkg.workloads.features(n, ci, 1)).to(dev)
+    w = torch.from_numpy(pkg.workloads.conv_weight(co, ci, 2)).to(dev)
+    b = torch.linspace(-1, 1, co, device=dev)
+    r = torch.from_numpy(pkg.workloads.features(n, co, 3)).to(dev)
+    want = _conv64(f, w, b, nbr)
+    out = pkg.sparse_conv3d(f, w, b, nbr)
+    assert ((out.double() - want).norm() / want.norm()).item() <= 4e-6
+    res = pkg.sparse_conv3d(f, w, b, nbr, epilogue="residual", residual=r)
+    assert ((res.double() - want - r).norm() / want.norm()).item() <= 4e-6
+    ctx = pkg._lib.context(dev.index)
+    P = lambda t: t.data_ptr()
+    got = r.clone()
+    pkg._lib.check(ctx.lib.tsc_conv_fused_noalloc(
+        ctx.bind(), pkg._lib.TSC_F32, P(f), P(w), P(b), P(nbr), None, n, ci, co,
+        pkg._lib.TSC_EPI_BIAS_RESIDUAL, P(got), None, None, 0.0, P(got)))
+    assert torch.equal(got, res)
+
+
+@pytest.mark.parametrize("n,ci,co,misaligned", [(300, 32, 64, False), (33000, 48, 64, False),
+                                                (300, 64, 96, False), (300, 64, 64, True)])
+def test_conv_fp32_split_extreme_values(pkg, dev, n, ci, co, misaligned):
+    """Infinities, NaN and values whose nearest bf16 is infinite have no split into bf16 pieces:
+    their outputs are what fp32 arithmetic gives, and all others are unchanged."""
+    print(f"  conv fp32 extremes N={n} {ci}->{co}", flush=True)
+    nbr = torch.from_numpy(_random_table(n, 7, 0.3)).to(dev)
+    f = torch.from_numpy(pkg.workloads.features(n, ci, 1)).to(dev)
+    w = torch.from_numpy(pkg.workloads.conv_weight(co, ci, 2)).to(dev)
+    b = torch.zeros(co, device=dev)
+    put = (lambda t: _offset(t)) if misaligned else (lambda t: t)
+    plain = pkg.sparse_conv3d(put(f), put(w), put(b), nbr)
+    f[5, 3], f[17, 0], f[40, ci - 1] = float("inf"), float("nan"), -3.4e38
+    f[77, ci // 2] = float("-inf")
+    out = pkg.sparse_conv3d(put(f), put(w), put(b), nbr)
+    want = _conv64(f, w, b, nbr)
+    f32max = torch.finfo(torch.float32).max
+    assert torch.equal(out.isnan(), want.isnan())
+    inf = want.isinf()
+    assert torch.equal(out[inf].double(), want[inf])
+    hit = torch.isin(nbr, torch.tensor([5, 17, 40, 77], device=dev, dtype=torch.int32)).any(dim=1)
+    assert torch.equal(out[~hit], plain[~hit])
+    big = hit[:, None] & want.isfinite() & (want.abs() < f32max)
+    assert big.any()
+    assert ((out[big].double() - want[big]).abs() <= 1e-5 * want[big].abs().clamp_min(1.0)).all()

@@ -1181,6 +1181,352 @@ int launch_narrow(tsc_ctx* ctx, const ConvArgs& a) {
   return check_hip(hipGetLastError(), "conv launch");
 }
 
+// fp32 rows of 16 inputs and more on the bf16 matrix cores.
+//
+// v_mfma_f32_32x32x2_f32 runs at 1/16 of the bf16 rate, so an fp32 product as six bf16 ones is
+// 2.7x as fast.  x = x0 + x1 + x2, each the bf16 nearest to what the ones before left over: 24 bits
+// and both signs, so the sum is x itself (x2 loses bits only where |x| is below 2^-109).  Of the
+// nine products x_i w_j the three with i + j > 2 are left out: each is below 2^-25 of x w, less
+// than the rounding of the sums.  All are summed in fp32 by the MFMAs, of every 16 inputs the
+// smallest first.  Error against fp64 (rel. 2-norm, N(0,1) rows), fp32 MFMAs / this: 64->64
+// 5.9e-7 / 5.0e-7, 128->256 8.2e-7 / 7.1e-7, 512->512 1.7e-6 / 1.5e-6.  An infinite or NaN operand
+// (or one that rounds to an infinite bf16) has no such split; it always leaves an infinite or
+// NaN sum, and those outputs are summed again on fp32 MFMAs (split_redo).
+
+// 8 fp32 -> 3 x 8 bf16.
+__device__ __forceinline__ void split8(const float (&x)[8], uint4 (&out)[3]) {
+  typedef __bf16 bf16x2_t __attribute__((__vector_size__(4)));
+  uint32_t w[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = x[2 * i], b = x[2 * i + 1];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      const bf16x2_t v = {(__bf16)a, (__bf16)b};
+      w[p][i] = __builtin_bit_cast(uint32_t, v);
+      a -= __uint_as_float(w[p][i] << 16);
+      b -= __uint_as_float(w[p][i] & 0xffff0000u);
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < 3; ++p) out[p] = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
+}
+
+// acc[j] += a * b[j]: the pieces' products, smallest first.
+template <int FN>
+__device__ __forceinline__ void split_mma(const uint4 (&a)[3], const uint4 (&b)[FN][3],
+                                          f32x16_t (&acc)[FN]) {
+#pragma unroll
+  for (int q = 2; q >= 0; --q)
+#pragma unroll
+    for (int p = q; p >= 0; --p)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) mfma_piece<__bf16>(a[p], b[j][q - p], acc[j]);
+}
+
+// Whether a sum of this wave is infinite or NaN.
+template <int FN>
+__device__ __forceinline__ bool split_bad(const f32x16_t (&acc)[FN]) {
+  float z = 0.f;
+#pragma unroll
+  for (int j = 0; j < FN; ++j)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) z = fmaf(acc[j][e], 0.f, z);
+  return __any(z != 0.f);  // NaN compares unequal
+}
+
+// The sums that are not finite, again on fp32 operands straight from memory.  nbr27: this lane's
+// row's 27 neighbors; w: this lane's column's 27 rows of Ci weights.
+__device__ __forceinline__ void split_redo(const float* feats, const float* w,
+                                           const int32_t* nbr27, uint32_t taps, int32_t Ci,
+                                           f32x16_t& acc) {
+  const int hf = (threadIdx.x & 63) >> 5;
+  f32x16_t again;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) again[e] = 0.f;
+  for (; taps; taps &= taps - 1) {
+    const int v = __ffs(taps) - 1;
+    const int32_t src = nbr27[v];
+    const float* ap = src >= 0 ? feats + (int64_t)src * Ci : (const float*)g_zero;
+    const float* bp = w + (int64_t)v * Ci;
+    for (int k = hf; k < Ci; k += 2)
+      again = __builtin_amdgcn_mfma_f32_32x32x2f32(ap[k], bp[k], again, 0, 0, 0);
+  }
+#pragma unroll
+  for (int e = 0; e < 16; ++e)
+    if (acc[e] * 0.f != 0.f) acc[e] = again[e];
+}
+
+// weight (rows, Ci) fp32 -> (rows, Ci / 16, 3, 16) bf16; thread = 8 consecutive inputs.
+constexpr int kSplitThreads = 256;
+__global__ void __launch_bounds__(kSplitThreads)
+    split_weights_kernel(const float* __restrict__ weight, int64_t n8, uint4* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * kSplitThreads + threadIdx.x;
+  if (i >= n8) return;
+  const float4 u = ((const float4*)weight)[2 * i], v = ((const float4*)weight)[2 * i + 1];
+  const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+  uint4 p[3];
+  split8(x, p);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) out[(i >> 1) * 6 + 2 * k + (i & 1)] = p[k];
+}
+
+// LDS swizzle of a split weight row (6 pieces of 16 bytes): 16 consecutive lanes read one piece of
+// 16 consecutive rows, which without it start in 8 of the 16 bank groups.
+__device__ __forceinline__ int swz_split(int row, int part) { return part ^ ((row >> 3) & 1); }
+
+// WM waves of 32 rows x 32 FN columns.  A row is used by one wave only, so its inputs go from
+// memory to that wave's registers, AHEAD chunks of 16 inputs early, and are split there; the
+// weights of the tap's chunk come into an LDS ring as in conv_mfma_kernel, already split
+// (WSPLIT: by split_weights_kernel) or split by every wave, with the same results, where there is
+// no buffer for that.  Only weights pass through LDS, so four blocks share a CU and their loads,
+// splits and MFMAs overlap: with the rows in the ring as well (two blocks) the three added up.
+// Loads are unconditional (past the end: the last weights again, zero rows): with branches
+// around them the compiler waits for every load in flight before the first use of a row.
+// Bound: the bf16 matrix rate at what the chip's power allows (800 of the 1300 TFLOP/s that a
+// large bf16 product reaches here, with 12-67 % more taps than the rows have).  Against the
+// fp32 MFMA ring kernel this replaced: 32->64 on 1.5 M voxels 745 -> 582 us, 64->64 on 300 k
+// 466 -> 340, 64->64 on 25 k 73 -> 61, 128->256 on 40 k 588 -> 410, 512->512 on 10 k 1494 -> 871.
+// Splitting the next chunk's rows beside the MFMAs: 1-5 % slower.  32 x 128 per wave: 300->288 us
+// to 871->923 as the tiles fill the CUs.
+template <int WM, int FN, int STAGES, int AHEAD, bool WSPLIT, int EPI>
+__global__ void __launch_bounds__(64 * WM, WM * FN == 8 ? 4 : 1)
+    conv_split_kernel(const float* __restrict__ feats, const float* __restrict__ weight,
+                      const uint4* __restrict__ wsplit, const float* __restrict__ bias,
+                      const int32_t* __restrict__ nbr, const int32_t* __restrict__ order,
+                      int64_t N, int32_t Ci, int32_t Co, int32_t m_tiles, int32_t n_tiles,
+                      int32_t per_xcd, const float* residual, float* out) {
+  constexpr int BM = 32 * WM, BN = 32 * FN, NT = 64 * WM;
+  constexpr int PPRB = WSPLIT ? 6 : 4;       // 16-byte pieces per weight row and chunk
+  constexpr int SB = BN * PPRB * 16;         // bytes per stage
+  constexpr int PPW = BN * PPRB / WM;        // pieces per wave
+  constexpr int IPW = (PPW + 63) / 64;       // loads per wave
+  static_assert(BN * PPRB % WM == 0, "every wave issues the same loads");
+  __shared__ __attribute__((aligned(16))) unsigned char ring[STAGES * SB];
+  __shared__ int32_t sNbr[BM * kTaps];
+  __shared__ int32_t sRow[BM];
+  __shared__ uint32_t sMask;
+
+  int m_tile, n_tile;
+  if (!tile_of(blockIdx.x, m_tiles, n_tiles, per_xcd, nullptr, &m_tile, &n_tile)) return;
+  const int64_t m0 = (int64_t)m_tile * BM;
+  const int n0 = n_tile * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, l32 = lane & 31, hf = lane >> 5;
+
+  if (tid == 0) sMask = 0u;
+  for (int r = tid; r < BM; r += NT) {
+    const int64_t pos = m0 + r;
+    sRow[r] = (pos < N) ? (order ? order[pos] : (int32_t)pos) : -1;
+  }
+  __syncthreads();
+  uint32_t mymask = load_tile_nbr<BM * kTaps, NT>(nbr, sRow, sNbr, tid);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) mymask |= __shfl_xor(mymask, off, 64);
+  if (lane == 0 && mymask) atomicOr(&sMask, mymask);
+  __syncthreads();
+  const uint32_t mask = __builtin_amdgcn_readfirstlane(sMask);
+  const int cpt = Ci / 16;                    // chunks per tap
+  const int nchunks = __popc(mask) * cpt;
+
+  f32x16_t acc[FN];
+#pragma unroll
+  for (int j = 0; j < FN; ++j)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[j][e] = 0.f;
+
+  // Row loads: chunk after chunk, inputs 16k + 8hf .. + 7 of this lane's row.
+  const int myrow = wid * 32 + l32;
+  uint32_t am = mask;
+  int ak = cpt - 1;
+  const float* ap = (const float*)g_zero;
+  auto load_a = [&](float (&x)[8]) {
+    if (++ak == cpt) {  // uniform
+      ak = 0;
+      int32_t src = -1;
+      if (am) {
+        src = lds_read_i32(sNbr + myrow * kTaps + (__ffs(am) - 1));
+        lds_wait_all();
+        pin(src);
+        am &= am - 1;
+      }
+      ap = (src >= 0 ? feats + (int64_t)src * Ci : (const float*)g_zero) + 8 * hf;
+    }
+    const float4 u = *(const float4*)(ap + 16 * ak), v = *(const float4*)(ap + 16 * ak + 4);
+    x[0] = u.x; x[1] = u.y; x[2] = u.z; x[3] = u.w;
+    x[4] = v.x; x[5] = v.y; x[6] = v.z; x[7] = v.w;
+  };
+  // Weight loads into ring stage bstage; past the last chunk the last one again.
+  uint32_t bm = mask;
+  int bk = 0, bv = mask ? __ffs(mask) - 1 : 0, bstage = 0;
+  uint32_t boff[IPW];
+#pragma unroll
+  for (int j = 0; j < IPW; ++j) {
+    const int L = min(wid * PPW + j * 64 + lane, BN * PPRB - 1), r = L / PPRB, pc = L % PPRB;
+    boff[j] = (uint32_t)r * kTaps * cpt * (PPRB * 16) +
+              (WSPLIT ? swz_split(r, pc) : swz<4>(r, pc)) * 16;
+  }
+  const char* const bbase = (WSPLIT ? (const char*)wsplit : (const char*)weight) +
+                            (int64_t)n0 * kTaps * cpt * (PPRB * 16);
+  auto load_b = [&]() {
+    const char* base = bbase + (int64_t)(bv * cpt + bk) * (PPRB * 16);
+#pragma unroll
+    for (int j = 0; j < IPW; ++j)
+      if (PPW % 64 == 0 || j * 64 + lane < PPW)
+        lds_dma16(base + boff[j], (lds_ptr_t)(ring + bstage * SB + (wid * PPW + j * 64) * 16));
+    bstage = bstage + 1 == STAGES ? 0 : bstage + 1;
+    if (bk + 1 < cpt) {
+      ++bk;
+    } else if (bm & (bm - 1)) {
+      bm &= bm - 1;
+      bv = __ffs(bm) - 1;
+      bk = 0;
+    }
+  };
+
+  const uint32_t ring0 = lds_addr(ring);
+  int rstage = 0;
+  auto step = [&](float (&x)[8]) {
+    // This wave's part of the chunk is in LDS: at most the loads of the STAGES - 2 chunks after it
+    // are in flight (row loads in flight only make the wait longer).  After the barrier
+    // every wave's is, and every wave has read the stage that load_b refills.
+    wait_vmcnt<IPW * (STAGES - 2)>();
+    TSC_COMPILER_BARRIER();
+    __builtin_amdgcn_s_barrier();
+    TSC_COMPILER_BARRIER();
+    uint4 as[3];
+    split8(x, as);
+    load_a(x);
+    load_b();
+    const uint32_t b0 = ring0 + rstage * SB;
+    rstage = rstage + 1 == STAGES ? 0 : rstage + 1;
+    constexpr int NP = WSPLIT ? 3 : 2;
+    u32x4 br[FN][NP];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int r = j * 32 + l32;
+#pragma unroll
+      for (int p = 0; p < NP; ++p)
+        br[j][p] = lds_read16(b0 + (r * PPRB + (WSPLIT ? swz_split(r, 2 * p + hf)
+                                                       : swz<4>(r, 2 * hf + p))) * 16);
+    }
+    lds_wait_all();
+    uint4 bs[FN][3];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+#pragma unroll
+      for (int p = 0; p < NP; ++p) pin(br[j][p]);
+      if constexpr (WSPLIT) {
+#pragma unroll
+        for (int p = 0; p < 3; ++p) bs[j][p] = __builtin_bit_cast(uint4, br[j][p]);
+      } else {
+        float w[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) w[e] = __uint_as_float(br[j][e >> 2][e & 3]);
+        split8(w, bs[j]);
+      }
+    }
+    split_mma<FN>(as, bs, acc);
+  };
+
+  if (nchunks > 0) {
+    float x[AHEAD][8];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) load_a(x[i]);
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s) load_b();
+    for (int c = 0; c < nchunks; c += AHEAD) {
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) step(x[i]);
+    }
+  }
+  wait_vmcnt<0>();  // weight loads past the end still write LDS
+
+  const int col = n0 + l32;
+  if (split_bad<FN>(acc)) {  // wave-uniform
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+      split_redo(feats, weight + (int64_t)(col + 32 * j) * kTaps * Ci, sNbr + myrow * kTaps, mask,
+                 Ci, acc[j]);
+  }
+
+  // A store writes 32 consecutive columns of two rows.  Residual values first: all loads before
+  // the first store (an output may alias the residual element by element).
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const int co = col + 32 * j;
+    const float bias_c = bias ? bias[co] : 0.f;
+    float rv[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      rv[e] = 0.f;
+      if (EPI == TSC_EPI_BIAS_RESIDUAL) {
+        const int32_t row = sRow[wid * 32 + 8 * (e >> 2) + 4 * hf + (e & 3)];
+        rv[e] = residual[(int64_t)(row >= 0 ? row : 0) * Co + co];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int32_t row = sRow[wid * 32 + 8 * (e >> 2) + 4 * hf + (e & 3)];
+      if (row < 0) continue;
+      float val = acc[j][e] + bias_c;
+      if (EPI == TSC_EPI_BIAS_RESIDUAL) val += rv[e];
+      out[(int64_t)row * Co + co] = val;
+    }
+  }
+}
+
+// The shapes conv_split_kernel takes (of those the tuned kernels take): every fp32 row of a
+// multiple of 16 inputs, except the narrow ones that have kernels of their own.
+inline bool split_shape(const ConvArgs& a) {
+  return a.dtype == TSC_F32 && a.Ci % 16 == 0 && a.Ci > 16 && a.Co % 32 == 0 &&
+         !(a.Ci == 32 && a.Co == 32);
+}
+
+// Weights split beforehand, or without a buffer for them (calls that may not allocate, captured
+// calls, whose graph would keep the address, more than kSplitMaxBytes, and a failed allocation)
+// in the kernel: the same results.
+constexpr int64_t kSplitMaxBytes = (int64_t)256 << 20;
+
+template <int WM, int FN, int STAGES, int AHEAD, int EPI>
+int launch_split(tsc_ctx* ctx, const ConvArgs& a) {
+  void* buf = nullptr;
+  const int64_t n8 = (int64_t)a.Co * kTaps * a.Ci / 8;
+  bool wsplit = !a.sched_scratch && n8 * 48 <= kSplitMaxBytes;
+  if (wsplit) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) {
+      (void)hipGetLastError();
+      cap = hipStreamCaptureStatusActive;
+    }
+    wsplit = cap == hipStreamCaptureStatusNone &&
+             split_workspace(ctx, (size_t)n8 * 48, &buf) == TSC_OK;
+  }
+  if (wsplit) {
+    ProfScope p(ctx, "conv_split_weights");
+    split_weights_kernel<<<(unsigned)((n8 + kSplitThreads - 1) / kSplitThreads), kSplitThreads, 0,
+                           ctx->stream>>>((const float*)a.weight, n8, (uint4*)buf);
+  }
+  const int32_t m_tiles = (int32_t)((a.N + 32 * WM - 1) / (32 * WM));
+  const int32_t n_tiles = a.Co / (32 * FN);
+  const int32_t per_xcd = tile_grid_per_xcd(m_tiles, n_tiles);
+  static const std::string base = "conv_split_kernel<" + std::to_string(32 * WM) + "x" +
+                                  std::to_string(32 * FN);
+  static const std::string names[2] = {
+      base + ",ab" + (EPI == TSC_EPI_BIAS_RESIDUAL ? ",res>" : ">"),
+      base + (EPI == TSC_EPI_BIAS_RESIDUAL ? ",res>" : ">")};
+  ProfScope p(ctx, names[wsplit].c_str());
+  auto run = [&](auto ws) {
+    conv_split_kernel<WM, FN, STAGES, AHEAD, decltype(ws)::value, EPI>
+        <<<(unsigned)per_xcd * 8u, 64 * WM, 0, ctx->stream>>>(
+            (const float*)a.feats, (const float*)a.weight, (const uint4*)buf,
+            (const float*)a.bias, a.nbr, a.order, a.N, a.Ci, a.Co, m_tiles, n_tiles, per_xcd,
+            (const float*)a.residual, (float*)a.out);
+  };
+  if (wsplit) run(std::true_type());
+  else run(std::false_type());
+  return check_hip(hipGetLastError(), "conv launch");
+}
+
 // Any channel counts (the reference bounds-checks Ci and Co, conv3d_wgsl.ts:174-196, so it takes
 // any shape): 64-row x 64-column tiles of four 32x32 waves, K in chunks of 32 bytes per row.
 // Each chunk is loaded into registers in pieces of LW bytes (the widest width that divides the
@@ -1195,9 +1541,11 @@ template <> struct PieceOf<4> { typedef uint32_t type; };
 template <> struct PieceOf<8> { typedef uint2 type; };
 template <> struct PieceOf<16> { typedef uint4 type; };
 
-constexpr int kGenBM = 64, kGenBN = 64, kGenKB = 32, kGenThreads = 256;
+constexpr int kGenBM = 64, kGenBN = 64, kGenThreads = 256;
 
-template <typename T, int LW, int EPI>
+// SPLIT: shapes of conv_split_kernel in buffers that are not 16-byte aligned: its arithmetic, in its
+// chunks of 64 bytes, so that alignment does not change a result.
+template <typename T, int LW, int EPI, bool SPLIT>
 __global__ void __launch_bounds__(kGenThreads)
     conv_generic_kernel(const T* __restrict__ feats, const T* __restrict__ weight,
                         const T* __restrict__ bias, const int32_t* __restrict__ nbr,
@@ -1205,7 +1553,7 @@ __global__ void __launch_bounds__(kGenThreads)
                         int32_t m_tiles, int32_t n_tiles, int32_t per_xcd, const T* residual,
                         T* out) {
   typedef typename PieceOf<LW>::type P;
-  constexpr int BM = kGenBM, BN = kGenBN, KB = kGenKB, NT = kGenThreads;
+  constexpr int BM = kGenBM, BN = kGenBN, KB = SPLIT ? 64 : 32, NT = kGenThreads;
   constexpr int EPL = LW / (int)sizeof(T);  // elements per piece
   constexpr int KC = KB / (int)sizeof(T);   // elements per chunk
   constexpr int LPR = KB / LW;              // pieces per row per chunk
@@ -1281,10 +1629,10 @@ __global__ void __launch_bounds__(kGenThreads)
       rb[j] = val;
     }
   };
-  // Piece k of row r sits at byte k*LW of the row's 32 bytes; its 16-byte half is swizzled.
+  // Piece k of row r sits at byte k*LW of the row's chunk, whose 16-byte parts are swizzled.
   auto lds_off = [](int r, int k) {
     const int byte = k * LW;
-    return r * KB + swz<2>(r, byte >> 4) * 16 + (byte & 15);
+    return r * KB + swz<KB / 16>(r, byte >> 4) * 16 + (byte & 15);
   };
   auto store_chunk = [&](int buf) {
 #pragma unroll
@@ -1309,14 +1657,33 @@ __global__ void __launch_bounds__(kGenThreads)
     const int buf = c & 1;
     __syncthreads();
     if (c + 1 < nchunks) load_chunk(c + 1);
-    const uint4 a = *(const uint4*)(&sA[buf][ar * KB + swz<2>(ar, part) * 16]);
-    const uint4 b = *(const uint4*)(&sB[buf][br * KB + swz<2>(br, part) * 16]);
-    mfma_piece<T>(a, b, acc);
+    if constexpr (SPLIT) {
+      uint4 as[3], bs[1][3];
+      auto split_row = [&](const unsigned char* row, int r, uint4(&o)[3]) {
+        float x[8];
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+          *(float4*)(x + 4 * k) = *(const float4*)(row + r * KB + swz<4>(r, 2 * part + k) * 16);
+        split8(x, o);
+      };
+      split_row(sA[buf], ar, as);
+      split_row(sB[buf], br, bs[0]);
+      split_mma<1>(as, bs, *(f32x16_t(*)[1])&acc);
+    } else {
+      const uint4 a = *(const uint4*)(&sA[buf][ar * KB + swz<2>(ar, part) * 16]);
+      const uint4 b = *(const uint4*)(&sB[buf][br * KB + swz<2>(br, part) * 16]);
+      mfma_piece<T>(a, b, acc);
+    }
     if (c + 1 < nchunks) store_chunk(buf ^ 1);
   }
 
   const int co = n0 + wn * 32 + (lane & 31);
   if (co >= Co) return;
+  if constexpr (SPLIT) {
+    if (split_bad<1>(*(const f32x16_t(*)[1])&acc))
+      split_redo((const float*)feats, (const float*)weight + (int64_t)co * kTaps * Ci,
+                 sNbr + ar * kTaps, mask, Ci, acc);
+  }
   const float bv = bias ? to_f32<T>(bias[co]) : 0.f;
   // Residual values first, all loads before the first store (see conv_regstage_kernel).
   float rv[16];
@@ -1339,19 +1706,26 @@ __global__ void __launch_bounds__(kGenThreads)
   }
 }
 
-template <typename T, int LW, int EPI>
-int launch_generic(tsc_ctx* ctx, const ConvArgs& a) {
+template <typename T, int LW, int EPI, bool SPLIT>
+int launch_generic_as(tsc_ctx* ctx, const ConvArgs& a) {
   const int32_t m_tiles = (int32_t)((a.N + kGenBM - 1) / kGenBM);
   const int32_t n_tiles = (a.Co + kGenBN - 1) / kGenBN;
   const int32_t per_xcd = tile_grid_per_xcd(m_tiles, n_tiles);
   static const std::string name = std::string("conv_generic_kernel<") +
       (sizeof(T) == 4 ? "f32" : std::is_same<T, __bf16>::value ? "bf16" : "f16") + ",p" +
-      std::to_string(LW) + (EPI == TSC_EPI_BIAS_RESIDUAL ? ",res>" : ">");
+      std::to_string(LW) + (SPLIT ? ",split" : "") + (EPI == TSC_EPI_BIAS_RESIDUAL ? ",res>" : ">");
   ProfScope p(ctx, name.c_str());
-  conv_generic_kernel<T, LW, EPI><<<(unsigned)per_xcd * 8u, kGenThreads, 0, ctx->stream>>>(
+  conv_generic_kernel<T, LW, EPI, SPLIT><<<(unsigned)per_xcd * 8u, kGenThreads, 0, ctx->stream>>>(
       (const T*)a.feats, (const T*)a.weight, (const T*)a.bias, a.nbr, a.order, a.N, a.Ci, a.Co,
       m_tiles, n_tiles, per_xcd, (const T*)a.residual, (T*)a.out);
   return check_hip(hipGetLastError(), "conv launch");
+}
+
+template <typename T, int LW, int EPI>
+int launch_generic(tsc_ctx* ctx, const ConvArgs& a) {
+  if constexpr (sizeof(T) == 4)
+    if (split_shape(a)) return launch_generic_as<T, LW, EPI, true>(ctx, a);
+  return launch_generic_as<T, LW, EPI, false>(ctx, a);
 }
 
 template <typename T, int EPI>
@@ -1415,15 +1789,24 @@ int dispatch_tiles(tsc_ctx* ctx, const ConvArgs& a) {
       return launch_cfg<T, 128, 64, 32, 4, 1, EPI>(ctx, a);
     }
   } else {
-    // Small problems (fewer 128-row tiles than CUs, e.g. ~25k voxels): 64x64 tiles of four
-    // 32x32 waves so every CU gets work.
-    if (a.Co % 64 == 0 && kb >= 128 && ((a.N + 127) / 128) * (a.Co / 64) < 256)
-      return launch_cfg<T, 64, 64, 128, 2, 2, EPI>(ctx, a);
-    if (a.Co % 64 == 0 && kb >= 64) return launch_cfg<T, 128, 64, 64, 4, 1, EPI>(ctx, a);
+    if (split_shape(a)) {
+      if (a.Co % 64 != 0) return launch_split<4, 1, 4, 2, EPI>(ctx, a);
+      // Fewer 128 x 64 tiles than CUs (e.g. 25 k voxels of 64 channels): 64 x 64 tiles, or still
+      // fewer than CUs, 64 x 32, each with a deeper pipeline, since few blocks share a CU.
+      // 64->64: 25 k voxels 77 / 67 / 75 us in 128 x 64 / 64 x 64 / 64 x 32 tiles, 3 k 61 / 60 / 50.
+      const int64_t n64 = a.Co / 64;
+      if ((a.N + 127) / 128 * n64 < 256)
+        return (a.N + 63) / 64 * n64 < 256 ? launch_split<2, 1, 8, 4, EPI>(ctx, a)
+                                           : launch_split<2, 2, 8, 4, EPI>(ctx, a);
+      return launch_split<4, 2, 4, 2, EPI>(ctx, a);
+    }
+    return launch_cfg<T, 128, 32, 32, 4, 1, EPI>(ctx, a);
   }
   // Co % 32 == 0
-  if (kb >= 64) return launch_cfg<T, 128, 32, 64, 4, 1, EPI>(ctx, a);
-  return launch_cfg<T, 128, 32, 32, 4, 1, EPI>(ctx, a);
+  if constexpr (sizeof(T) < 4) {
+    if (kb >= 64) return launch_cfg<T, 128, 32, 64, 4, 1, EPI>(ctx, a);
+    return launch_cfg<T, 128, 32, 32, 4, 1, EPI>(ctx, a);
+  }
 }
 
 // The ring configurations of dispatch_tiles whose column tile is the whole row (BN == Co), with
