@@ -515,3 +515,31 @@ def test_conv_fp32_split_extreme_values(pkg, dev, n, ci, co, misaligned):
     big = hit[:, None] & want.isfinite() & (want.abs() < f32max)
     assert big.any()
     assert ((out[big].double() - want[big]).abs() <= 1e-5 * want[big].abs().clamp_min(1.0)).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,ci,co", [
+    (1, 64, 64), (65, 64, 256), (32768, 32 * 3, 64), (4096, 64, 512),  # 64 x 64, up to 512 tiles
+    (16385, 64, 128), (8193, 64, 256), (4097, 64, 512),                # 128 x 64 from there
+    (16385, 64, 256), (32769, 64, 256),                                # 128 x 128, 256 x 256
+    (32769, 64, 64), (32769, 64, 128)])
+def test_conv_tiles_by_grid_size(pkg, dev, dtype, n, ci, co):
+    """Either side of each size at which the 16-bit convs change their tile, with every epilogue.
+    A result is a sum in fp32 rounded once: within half a unit in the last place (2^-9 / 2^-12 of the
+    value) of fp64, and the sums' own errors are below a tenth of that."""
+    print(f"  conv tiles N={n} {ci}->{co} {dtype}", flush=True)
+    nbr = torch.from_numpy(_random_table(n, n)).to(dev)
+    f = torch.from_numpy(pkg.workloads.features(n, ci, 1)).to(dev).to(dtype)
+    w = torch.from_numpy(pkg.workloads.conv_weight(co, ci, 2)).to(dev).to(dtype)
+    b = torch.linspace(-1, 1, co, device=dev).to(dtype)
+    r = torch.from_numpy(pkg.workloads.features(n, co, 3)).to(dev).to(dtype)
+    tol = 1.1 * (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12)
+    want = _conv64(f, w, b, nbr)
+    out = pkg.sparse_conv3d(f, w, b, nbr)
+    assert ((out.double() - want).norm() / want.norm()).item() <= tol
+    res = pkg.sparse_conv3d(f, w, b, nbr, epilogue="residual", residual=r)
+    want = want + r.double()
+    assert ((res.double() - want).norm() / want.norm()).item() <= tol
+    g = torch.linspace(0.5, 1.5, co, device=dev).to(dtype)
+    ln = pkg.sparse_conv3d(f, w, b, nbr, epilogue="ln_silu", ln_weight=g, ln_bias=b)
+    assert torch.equal(ln, pkg.layer_norm(out, g, b, silu=True))

@@ -1774,20 +1774,29 @@ int dispatch_tiles(tsc_ctx* ctx, const ConvArgs& a) {
   // stage 32 epilogue rows of a 128-column half tile or a 64-column fp32 tile, so those shapes
   // take the next narrower tile.
   if constexpr (sizeof(T) < 4) {
-    if (a.Co % 256 == 0 && kb >= 64) {
+    if (a.Co % 64 == 0 && kb >= 64) {
+      // The smallest tile of which every one has its place on the chip at once (two blocks per
+      // CU).  A tile's time is its chain of K chunks, so while CUs are left over smaller tiles,
+      // whose chunks take less, end sooner; past that the larger ones' reuse of rows and weights
+      // wins.  us in 64x64 / 128x64 / 128x128 / 256x256 tiles (tiles):
+      //   256->256    2 k voxels    57  (128)   69   (64)    87   (32)   170   (8)
+      //   256->256   10 k          102  (628)   77  (316)    87  (158)   170  (40)
+      //   256->256   20 k          153 (1252)  144  (628)   116  (314)   169  (79)
+      //   512->512   20 k          488 (2504)  433 (1256)   389  (628)   332 (158)
+      //   1024->1024  2 k          241  (512)  251  (256)   307  (128)   620  (32)
+      auto tiles = [&](int bm, int bn) { return (a.N + bm - 1) / bm * (a.Co / bn); };
+      constexpr int64_t kSlots = 512;
+      if (tiles(64, 64) <= kSlots) return launch_cfg<T, 64, 64, 64, 2, 2, EPI>(ctx, a);
+      if (a.Co % 128 != 0 || tiles(128, 64) <= kSlots)
+        return launch_cfg<T, 128, 64, 64, 4, 1, EPI>(ctx, a);  // 4 waves of 32 rows
+      // Wide channels: 128x128 tile, 2x2 waves of 64x64, two blocks per CU.
+      if (a.Co % 256 != 0 || tiles(128, 128) <= kSlots)
+        return launch_cfg<T, 128, 128, 64, 2, 2, EPI>(ctx, a);
       // Widest channels: 256x256 tile, 2x4 waves of 128x64, one block per CU with a 4-stage
       // ring (128 flops per LDS/L2 byte, 0.75 fragment reads per MFMA).
       return launch_cfg<T, 256, 256, 64, 2, 4, EPI, 1>(ctx, a);
     }
-    if (a.Co % 128 == 0 && kb >= 64) {
-      // Wide channels: 128x128 tile, 2x2 waves of 64x64, two blocks per CU.
-      return launch_cfg<T, 128, 128, 64, 2, 2, EPI>(ctx, a);
-    }
-    if (a.Co % 64 == 0) {
-      // 128 rows x 64 cols, 4 waves of 32 rows.
-      if (kb >= 64) return launch_cfg<T, 128, 64, 64, 4, 1, EPI>(ctx, a);
-      return launch_cfg<T, 128, 64, 32, 4, 1, EPI>(ctx, a);
-    }
+    if (a.Co % 64 == 0) return launch_cfg<T, 128, 64, 32, 4, 1, EPI>(ctx, a);
   } else {
     if (split_shape(a)) {
       if (a.Co % 64 != 0) return launch_split<4, 1, 4, 2, EPI>(ctx, a);
@@ -1815,10 +1824,16 @@ template <typename T>
 int dispatch_ln(tsc_ctx* ctx, const ConvArgs& a) {
   if constexpr (sizeof(T) == 2) {
     const int kb = pick_kb(a.Ci * 2);
+    // 64-row tiles while there is room for all of them, as in dispatch_tiles.
+    const bool few = (a.N + 63) / 64 <= 512 && kb >= 64;
     if (a.Co == 256 && kb >= 64)
-      return launch_cfg<T, 256, 256, 64, 2, 4, TSC_EPI_BIAS_LN_SILU, 1>(ctx, a);
-    if (a.Co == 128 && kb >= 64) return launch_cfg<T, 128, 128, 64, 2, 2, TSC_EPI_BIAS_LN_SILU>(ctx, a);
+      return few ? launch_cfg<T, 64, 256, 64, 2, 4, TSC_EPI_BIAS_LN_SILU>(ctx, a)
+                 : launch_cfg<T, 256, 256, 64, 2, 4, TSC_EPI_BIAS_LN_SILU, 1>(ctx, a);
+    if (a.Co == 128 && kb >= 64)
+      return few ? launch_cfg<T, 64, 128, 64, 2, 2, TSC_EPI_BIAS_LN_SILU>(ctx, a)
+                 : launch_cfg<T, 128, 128, 64, 2, 2, TSC_EPI_BIAS_LN_SILU>(ctx, a);
     if (a.Co == 64) {
+      if (few) return launch_cfg<T, 64, 64, 64, 2, 2, TSC_EPI_BIAS_LN_SILU>(ctx, a);
       if (kb >= 64) return launch_cfg<T, 128, 64, 64, 4, 1, TSC_EPI_BIAS_LN_SILU>(ctx, a);
       return launch_cfg<T, 128, 64, 32, 4, 1, TSC_EPI_BIAS_LN_SILU>(ctx, a);
     }
