@@ -543,3 +543,21 @@ def test_conv_tiles_by_grid_size(pkg, dev, dtype, n, ci, co):
     g = torch.linspace(0.5, 1.5, co, device=dev).to(dtype)
     ln = pkg.sparse_conv3d(f, w, b, nbr, epilogue="ln_silu", ln_weight=g, ln_bias=b)
     assert torch.equal(ln, pkg.layer_norm(out, g, b, silu=True))
+
+
+@pytest.mark.parametrize("dtype,ci,co", [(torch.bfloat16, 8, 64), (torch.float32, 6, 40),
+                                         (torch.float16, 20, 100), (torch.float32, 40, 72)])
+@pytest.mark.parametrize("n", [1, 63, 65, 32769, 65537])
+def test_conv_generic_by_grid_size(pkg, dev, dtype, ci, co, n):
+    """The generic kernel with four chunks in flight (up to 1024 tiles of 64 x 64) and with one, at
+    ragged widths of 8- and 16-byte pieces and chunk counts that are no multiple of four."""
+    print(f"  conv generic N={n} {ci}->{co} {dtype}", flush=True)
+    nbr = torch.from_numpy(_random_table(n, n)).to(dev)
+    f = torch.from_numpy(pkg.workloads.features(n, ci, 1)).to(dev).to(dtype)
+    w = torch.from_numpy(pkg.workloads.conv_weight(co, ci, 2)).to(dev).to(dtype)
+    b = torch.linspace(-1, 1, co, device=dev).to(dtype)
+    want = _conv64(f, w, b, nbr)
+    out = pkg.sparse_conv3d(f, w, b, nbr)
+    # one rounding of the result; fp32: of its sums (see test_conv_fp32_split_tiles)
+    tol = {torch.bfloat16: 1.1 * 2.0 ** -9, torch.float16: 1.1 * 2.0 ** -12, torch.float32: 4e-6}
+    assert ((out.double() - want).norm() / want.norm()).item() <= tol[dtype]

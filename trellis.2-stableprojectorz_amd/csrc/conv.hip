@@ -1545,7 +1545,7 @@ constexpr int kGenBM = 64, kGenBN = 64, kGenThreads = 256;
 
 // SPLIT: shapes of conv_split_kernel in buffers that are not 16-byte aligned: its arithmetic, in its
 // chunks of 64 bytes, so that alignment does not change a result.
-template <typename T, int LW, int EPI, bool SPLIT>
+template <typename T, int LW, int EPI, bool SPLIT, int AHEAD>
 __global__ void __launch_bounds__(kGenThreads)
     conv_generic_kernel(const T* __restrict__ feats, const T* __restrict__ weight,
                         const T* __restrict__ bias, const int32_t* __restrict__ nbr,
@@ -1599,64 +1599,16 @@ __global__ void __launch_bounds__(kGenThreads)
 #pragma unroll
   for (int e = 0; e < 16; ++e) acc[e] = 0.f;
 
-  P ra[AL], rb[BL];
   P zero;
   __builtin_memset(&zero, 0, sizeof(P));
-  auto load_chunk = [&](int c) {
-    const int ti = c / cpt;
-    const int ci0 = (c - ti * cpt) * KC;
-    const int v = sTaps[ti];
-#pragma unroll
-    for (int j = 0; j < AL; ++j) {
-      const int q = tid + j * NT;
-      P val = zero;
-      if (q < BM * LPR) {
-        const int r = q / LPR, ci = ci0 + (q % LPR) * EPL;
-        const int32_t src = sNbr[r * kTaps + v];
-        if (src >= 0 && ci < Ci) val = *(const P*)(feats + (int64_t)src * Ci + ci);
-      }
-      ra[j] = val;
-    }
-#pragma unroll
-    for (int j = 0; j < BL; ++j) {
-      const int q = tid + j * NT;
-      P val = zero;
-      if (q < BN * LPR) {
-        const int r = q / LPR, ci = ci0 + (q % LPR) * EPL;
-        if (n0 + r < Co && ci < Ci)
-          val = *(const P*)(weight + ((int64_t)(n0 + r) * kTaps + v) * Ci + ci);
-      }
-      rb[j] = val;
-    }
-  };
   // Piece k of row r sits at byte k*LW of the row's chunk, whose 16-byte parts are swizzled.
   auto lds_off = [](int r, int k) {
     const int byte = k * LW;
     return r * KB + swz<KB / 16>(r, byte >> 4) * 16 + (byte & 15);
   };
-  auto store_chunk = [&](int buf) {
-#pragma unroll
-    for (int j = 0; j < AL; ++j) {
-      const int q = tid + j * NT;
-      if (q < BM * LPR) *(P*)(&sA[buf][lds_off(q / LPR, q % LPR)]) = ra[j];
-    }
-#pragma unroll
-    for (int j = 0; j < BL; ++j) {
-      const int q = tid + j * NT;
-      if (q < BN * LPR) *(P*)(&sB[buf][lds_off(q / LPR, q % LPR)]) = rb[j];
-    }
-  };
-
-  if (nchunks > 0) {
-    load_chunk(0);
-    store_chunk(0);
-  }
   const int part = lane >> 5;
   const int ar = wm * 32 + (lane & 31), br = wn * 32 + (lane & 31);
-  for (int c = 0; c < nchunks; ++c) {
-    const int buf = c & 1;
-    __syncthreads();
-    if (c + 1 < nchunks) load_chunk(c + 1);
+  auto compute = [&](int buf) {
     if constexpr (SPLIT) {
       uint4 as[3], bs[1][3];
       auto split_row = [&](const unsigned char* row, int r, uint4(&o)[3]) {
@@ -1674,7 +1626,127 @@ __global__ void __launch_bounds__(kGenThreads)
       const uint4 b = *(const uint4*)(&sB[buf][br * KB + swz<2>(br, part) * 16]);
       mfma_piece<T>(a, b, acc);
     }
-    if (c + 1 < nchunks) store_chunk(buf ^ 1);
+  };
+  if constexpr (AHEAD > 1) {
+    // AHEAD chunks in flight into registers: absent pieces are loaded from row 0 and become zeros on
+    // their way into LDS, since a branch around a load would make the compiler wait for all loads
+    // in flight at the next use.
+    static_assert(AHEAD % 2 == 0 && AL <= 16 && BL <= 16, "buffer parity, present bits");
+    P ra[AHEAD][AL], rb[AHEAD][BL];
+    uint32_t ok[AHEAD];  // bit j: A piece j present, bit 16 + j: B piece j
+    uint32_t lm = mask;
+    int lk = 0;  // next chunk: Ci slice lk of the lowest tap in lm; past the end the last one again
+    auto load_chunk = [&](P(&xa)[AL], P(&xb)[BL], uint32_t& present) {
+      const int v = lm ? __ffs(lm) - 1 : 0, ci0 = lk * KC;
+      if (lk + 1 < cpt) {
+        ++lk;
+      } else if (lm & (lm - 1)) {
+        lm &= lm - 1;
+        lk = 0;
+      }
+      present = 0u;
+#pragma unroll
+      for (int j = 0; j < AL; ++j) {
+        const int q = min(tid + j * NT, BM * LPR - 1);
+        const int r = q / LPR, ci = ci0 + (q % LPR) * EPL;
+        const int32_t src = sNbr[r * kTaps + v];
+        const bool here = src >= 0 && ci < Ci;
+        present |= (uint32_t)here << j;
+        xa[j] = *(const P*)(feats + (here ? (int64_t)src * Ci + ci : 0));
+      }
+#pragma unroll
+      for (int j = 0; j < BL; ++j) {
+        const int q = min(tid + j * NT, BN * LPR - 1);
+        const int r = q / LPR, ci = ci0 + (q % LPR) * EPL;
+        const bool here = n0 + r < Co && ci < Ci;
+        present |= (uint32_t)here << (16 + j);
+        xb[j] = *(const P*)(weight + (here ? ((int64_t)(n0 + r) * kTaps + v) * Ci + ci : 0));
+      }
+    };
+    auto store_chunk = [&](int buf, const P(&xa)[AL], const P(&xb)[BL], uint32_t present) {
+#pragma unroll
+      for (int j = 0; j < AL; ++j) {
+        const int q = tid + j * NT;
+        P val = xa[j];
+        if (!(present >> j & 1u)) val = zero;
+        if (q < BM * LPR) *(P*)(&sA[buf][lds_off(q / LPR, q % LPR)]) = val;
+      }
+#pragma unroll
+      for (int j = 0; j < BL; ++j) {
+        const int q = tid + j * NT;
+        P val = xb[j];
+        if (!(present >> (16 + j) & 1u)) val = zero;
+        if (q < BN * LPR) *(P*)(&sB[buf][lds_off(q / LPR, q % LPR)]) = val;
+      }
+    };
+    if (nchunks > 0) {
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) load_chunk(ra[i], rb[i], ok[i]);
+      for (int c0 = 0; c0 < nchunks; c0 += AHEAD) {
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+          // Two LDS buffers, one barrier per chunk: every wave has read this buffer's last
+          // contents before the barrier of the chunk between.
+          store_chunk(i & 1, ra[i], rb[i], ok[i]);
+          __syncthreads();
+          load_chunk(ra[i], rb[i], ok[i]);
+          if (c0 + i < nchunks) compute(i & 1);  // uniform
+        }
+      }
+    }
+  } else {
+    P ra[AL], rb[BL];
+    auto load_chunk = [&](int c) {
+      const int ti = c / cpt;
+      const int ci0 = (c - ti * cpt) * KC;
+      const int v = sTaps[ti];
+#pragma unroll
+      for (int j = 0; j < AL; ++j) {
+        const int q = tid + j * NT;
+        P val = zero;
+        if (q < BM * LPR) {
+          const int r = q / LPR, ci = ci0 + (q % LPR) * EPL;
+          const int32_t src = sNbr[r * kTaps + v];
+          if (src >= 0 && ci < Ci) val = *(const P*)(feats + (int64_t)src * Ci + ci);
+        }
+        ra[j] = val;
+      }
+#pragma unroll
+      for (int j = 0; j < BL; ++j) {
+        const int q = tid + j * NT;
+        P val = zero;
+        if (q < BN * LPR) {
+          const int r = q / LPR, ci = ci0 + (q % LPR) * EPL;
+          if (n0 + r < Co && ci < Ci)
+            val = *(const P*)(weight + ((int64_t)(n0 + r) * kTaps + v) * Ci + ci);
+        }
+        rb[j] = val;
+      }
+    };
+    auto store_chunk = [&](int buf) {
+#pragma unroll
+      for (int j = 0; j < AL; ++j) {
+        const int q = tid + j * NT;
+        if (q < BM * LPR) *(P*)(&sA[buf][lds_off(q / LPR, q % LPR)]) = ra[j];
+      }
+#pragma unroll
+      for (int j = 0; j < BL; ++j) {
+        const int q = tid + j * NT;
+        if (q < BN * LPR) *(P*)(&sB[buf][lds_off(q / LPR, q % LPR)]) = rb[j];
+      }
+    };
+
+    if (nchunks > 0) {
+      load_chunk(0);
+      store_chunk(0);
+    }
+    for (int c = 0; c < nchunks; ++c) {
+      const int buf = c & 1;
+      __syncthreads();
+      if (c + 1 < nchunks) load_chunk(c + 1);
+      compute(buf);
+      if (c + 1 < nchunks) store_chunk(buf ^ 1);
+    }
   }
 
   const int co = n0 + wn * 32 + (lane & 31);
@@ -1706,7 +1778,7 @@ __global__ void __launch_bounds__(kGenThreads)
   }
 }
 
-template <typename T, int LW, int EPI, bool SPLIT>
+template <typename T, int LW, int EPI, bool SPLIT, int AHEAD>
 int launch_generic_as(tsc_ctx* ctx, const ConvArgs& a) {
   const int32_t m_tiles = (int32_t)((a.N + kGenBM - 1) / kGenBM);
   const int32_t n_tiles = (a.Co + kGenBN - 1) / kGenBN;
@@ -1715,7 +1787,7 @@ int launch_generic_as(tsc_ctx* ctx, const ConvArgs& a) {
       (sizeof(T) == 4 ? "f32" : std::is_same<T, __bf16>::value ? "bf16" : "f16") + ",p" +
       std::to_string(LW) + (SPLIT ? ",split" : "") + (EPI == TSC_EPI_BIAS_RESIDUAL ? ",res>" : ">");
   ProfScope p(ctx, name.c_str());
-  conv_generic_kernel<T, LW, EPI, SPLIT><<<(unsigned)per_xcd * 8u, kGenThreads, 0, ctx->stream>>>(
+  conv_generic_kernel<T, LW, EPI, SPLIT, AHEAD><<<(unsigned)per_xcd * 8u, kGenThreads, 0, ctx->stream>>>(
       (const T*)a.feats, (const T*)a.weight, (const T*)a.bias, a.nbr, a.order, a.N, a.Ci, a.Co,
       m_tiles, n_tiles, per_xcd, (const T*)a.residual, (T*)a.out);
   return check_hip(hipGetLastError(), "conv launch");
@@ -1724,8 +1796,16 @@ int launch_generic_as(tsc_ctx* ctx, const ConvArgs& a) {
 template <typename T, int LW, int EPI>
 int launch_generic(tsc_ctx* ctx, const ConvArgs& a) {
   if constexpr (sizeof(T) == 4)
-    if (split_shape(a)) return launch_generic_as<T, LW, EPI, true>(ctx, a);
-  return launch_generic_as<T, LW, EPI, false>(ctx, a);
+    if (split_shape(a)) return launch_generic_as<T, LW, EPI, true, 1>(ctx, a);
+  // While there are few tiles (all of them on the chip at once, or nearly) the chain of loads sets
+  // the time: four chunks in flight, if a load takes 8 bytes or more.  23 k voxels, 8->64 bf16
+  // (357 tiles): 15.2 -> 13.0 us; 40->72 (714) 37 -> 29, fp32 90 -> 77.  With more tiles the loads of
+  // absent pieces cost more than that gives (8->64 on 100 k, 1563: 24 -> 28), as with narrower
+  // loads (13->48, 2 k voxels: 25 -> 30).
+  if constexpr (LW >= 8)
+    if ((a.N + kGenBM - 1) / kGenBM * ((a.Co + kGenBN - 1) / kGenBN) <= 1024)
+      return launch_generic_as<T, LW, EPI, false, 4>(ctx, a);
+  return launch_generic_as<T, LW, EPI, false, 1>(ctx, a);
 }
 
 template <typename T, int EPI>
