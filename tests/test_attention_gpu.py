@@ -208,3 +208,28 @@ def test_key_counts_at_step_and_block_edges(pkg, dev, dtype, d, h):
     v[last] = float("inf")
     out = pkg.sparse_attention(q.to(dev), k.to(dev), v.to(dev), cu_q, cu_kv)
     assert bool((out == float("inf")).all())
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("step", [0.2, 3.0, -0.5])
+def test_attention_fp32_moving_maximum(pkg, dev, d, step):
+    """fp32 scores that rise (or fall) by about `step` from each key to the next, so that the running
+    maximum is raised within its headroom, in every block, or once; lengths around the 32-key blocks.
+    Scores reach 600, each off by up to 2^-24 of its terms' sum, and so is the probability's
+    exponent: 1e-4 of the result is twice that."""
+    lens = [1, 31, 32, 33, 200]
+    cu = np.cumsum([0] + lens).astype(np.int32)
+    g = torch.Generator().manual_seed(d)
+    q = torch.randn((cu[-1], 2, d), generator=g)
+    k = torch.randn((cu[-1], 2, d), generator=g)
+    v = torch.randn((cu[-1], 2, d), generator=g)
+    q[..., 0] = 1.0
+    for b, n in enumerate(lens):
+        k[cu[b]:cu[b + 1], :, 0] = step * torch.arange(n, dtype=torch.float32)[:, None]
+    print(f"  attention fp32 maximum D={d} step={step}", flush=True)
+    out = pkg.sparse_attention(q.to(dev), k.to(dev), v.to(dev), cu.tolist(), scale=1.0).cpu()
+    for b in range(len(lens)):
+        s = slice(cu[b], cu[b + 1])
+        p = torch.softmax(torch.einsum("qhd,khd->hqk", q[s].double(), k[s].double()), dim=2)
+        want = torch.einsum("hqk,khd->qhd", p, v[s].double())
+        assert ((out[s].double() - want).norm() / want.norm()).item() <= 1e-4
