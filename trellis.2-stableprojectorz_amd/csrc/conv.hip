@@ -10,7 +10,9 @@
 // valid-tap bits: taps that no row of the tile uses are skipped entirely.  The K loop then walks
 // (tap, Ci-chunk) pairs over XOR-swizzled LDS tiles of gathered A rows (feats[nbr[row,v]], zero
 // when nbr < 0) and K-contiguous B rows (W[co, v, ci-chunk]); four waves run 32x32 MFMAs
-// (v_mfma_f32_32x32x16_{bf16,f16}, v_mfma_f32_32x32x2_f32).  Two pipelines feed the tiles:
+// (v_mfma_f32_32x32x16_{bf16,f16}, v_mfma_f32_32x32x2_f32).  Three pipelines feed the tiles:
+//   conv_split_kernel     fp32 rows of a multiple of 16 inputs: three bf16 pieces per value, rows
+//                         straight to registers, split weights through a ring
 //   conv_mfma_kernel      rows longer than 64 bytes (wide channels, several chunks per tap):
 //                         a 3-8 stage ring filled by direct-to-LDS loads (global_load_lds),
 //                         per-tap source addresses kept in registers, fragments read with

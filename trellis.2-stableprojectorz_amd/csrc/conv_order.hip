@@ -288,14 +288,12 @@ __global__ void __launch_bounds__(kOrdThreads)
 constexpr int kGrChunk = 4096;   // rows per chunk (and at most this many entries)
 constexpr int kGrThreads = 512;
 constexpr int kGrTile = 256;     // rows per tile of the 256-row conv kernels
-// Sets of up to kFewRows rows (conv_order_few_launch): 1024-row chunks, so that a small set still
-// gives several blocks and each a quarter of the passes.
-constexpr int kGrFewChunk = 1024;
-constexpr int kGrFewThreads = 256;
 static_assert(kOrdTilesPerWin * kOrdTile % kGrChunk == 0, "chunks never straddle a window");
-static_assert(kGrTile <= kGrThreads && kGrTile <= kGrFewThreads, "one thread per tile slot");
+static_assert(kGrTile <= kGrThreads, "one thread per tile slot");
 
-constexpr uint32_t kSpent = 1u << 31;  // in an entry's mask: no rows left
+// In an entry's mask: no rows left.  Mask, next position and rows left are a register each: packed
+// into 64 bits, a pass spent its time unpacking (greedy pass at 6 k rows 121 against 98 us).
+constexpr uint32_t kSpent = 1u << 31;
 
 // Inclusive wave64 scans on DPP lane moves (row_shr inside each 16-lane row, then row_bcast:15
 // and row_bcast:31 across rows); lanes whose source is outside the row keep the identity.
