@@ -4,6 +4,8 @@ Tolerance (norm-wise relative, max|y - r| / max|r|, r computed in fp64 from the 
 inputs and weights): fp32 <= 1e-4, fp16 / bf16 <= 2e-2.  The workload convs also assert the
 per-element allclose with atol = rtol * rms(r) (tests/_tol.py) and print both.
 """
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -469,7 +471,7 @@ def test_conv_fp32_split_tiles(pkg, dev, n, ci, co):
     """fp32 convs on bf16 pieces, at the edges of every tile and with odd chunk counts per tap.  At
     most 27 Ci products are summed in fp32, each sum rounding by at most 2^-24 of its size: 4e-6
     of the result (2-norm) is some ten times the random walk of these roundings.  The same bits
-    from the noalloc entry, which splits the weights in the kernel, and in place on the residual."""
+    from the noalloc entry and in place on the residual."""
     print(f"  conv fp32 split N={n} {ci}->{co}", flush=True)
     nbr = torch.from_numpy(_random_table(n, n)).to(dev)
     f = torch.from_numpy(pkg.workloads.features(n, ci, 1)).to(dev)
@@ -561,3 +563,45 @@ def test_conv_generic_by_grid_size(pkg, dev, dtype, ci, co, n):
     # one rounding of the result; fp32: of its sums (see test_conv_fp32_split_tiles)
     tol = {torch.bfloat16: 1.1 * 2.0 ** -9, torch.float16: 1.1 * 2.0 ** -12, torch.float32: 4e-6}
     assert ((out.double() - want).norm() / want.norm()).item() <= tol[dtype]
+
+
+def test_conv_fp32_keeps_nothing_in_the_context(pkg, dev):
+    """An fp32 conv only enqueues: no device memory is taken (a copy of these weights in bf16 pieces
+    would be 170 MB) and nothing is left behind that the next conv on the context could meet."""
+    n, c = 300, 1024
+    nbr = torch.from_numpy(_random_table(n, 3)).to(dev)
+    f = torch.from_numpy(pkg.workloads.features(n, c, 1)).to(dev)
+    w = torch.from_numpy(pkg.workloads.conv_weight(c, c, 2)).to(dev)
+    out = torch.empty((n, c), device=dev)
+    small = torch.from_numpy(pkg.workloads.conv_weight(64, 64, 2)).to(dev)
+    pkg.sparse_conv3d(f[:, :64].contiguous(), small, None, nbr)  # the kernels' code is loaded
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info(dev)[0]
+    print("  conv fp32 device memory", flush=True)
+    pkg.sparse_conv3d(f, w, None, nbr, out=out)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info(dev)[0] < 32 << 20
+
+
+def test_conv_fp32_from_two_threads(pkg, dev):
+    """Two threads with weights of their own, on one stream: each gets its own results."""
+    n, c = 3000, 64
+    nbr = torch.from_numpy(_random_table(n, 3)).to(dev)
+    f = torch.from_numpy(pkg.workloads.features(n, c, 1)).to(dev)
+    ws = [torch.from_numpy(pkg.workloads.conv_weight(c, c, s)).to(dev) for s in (2, 3)]
+    want = [pkg.sparse_conv3d(f, w, None, nbr) for w in ws]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(i):
+        outs = [pkg.sparse_conv3d(f, ws[i], None, nbr) for _ in range(100)]
+        torch.cuda.synchronize()
+        wrong.extend(i for o in outs if not torch.equal(o, want[i]))
+
+    print("  conv fp32 two threads", flush=True)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong

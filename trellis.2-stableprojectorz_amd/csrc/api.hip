@@ -99,12 +99,6 @@ int blas_workspace(tsc_ctx* ctx, size_t bytes, void** out) {
   return grow_buffer(ctx, &ctx->ws_blas, &ctx->ws_blas_bytes, bytes, "hipBLASLt workspace", out);
 }
 
-int split_workspace(tsc_ctx* ctx, size_t bytes, void** out) {
-  const int st = grow_buffer(ctx, &ctx->ws_split, &ctx->ws_split_bytes, bytes, "split weights", out);
-  if (st) g_err[0] = 0;  // the conv does without
-  return st;
-}
-
 void prof_clear(tsc_ctx* ctx) {
   for (auto& r : ctx->prof) {
     (void)hipEventDestroy(r.start);
@@ -216,7 +210,6 @@ int tsc_ctx_destroy(tsc_ctx* ctx) {
     if (e.buf) (void)hipFree(e.buf);
   blas_destroy(ctx);
   if (ctx->ws_blas) (void)hipFree(ctx->ws_blas);
-  if (ctx->ws_split) (void)hipFree(ctx->ws_split);
   st_release(ctx);
   prof_clear(ctx);
   delete ctx;

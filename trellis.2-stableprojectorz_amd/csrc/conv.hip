@@ -12,7 +12,7 @@
 // when nbr < 0) and K-contiguous B rows (W[co, v, ci-chunk]); four waves run 32x32 MFMAs
 // (v_mfma_f32_32x32x16_{bf16,f16}, v_mfma_f32_32x32x2_f32).  Three pipelines feed the tiles:
 //   conv_split_kernel     fp32 rows of a multiple of 16 inputs: three bf16 pieces per value, rows
-//                         straight to registers, split weights through a ring
+//                         straight to registers, weights split on their way into LDS
 //   conv_mfma_kernel      rows longer than 64 bytes (wide channels, several chunks per tap):
 //                         a 3-8 stage ring filled by direct-to-LDS loads (global_load_lds),
 //                         per-tap source addresses kept in registers, fragments read with
@@ -1195,21 +1195,27 @@ int launch_narrow(tsc_ctx* ctx, const ConvArgs& a) {
 // (or one that rounds to an infinite bf16) has no such split; it always leaves an infinite or
 // NaN sum, and those outputs are summed again on fp32 MFMAs (split_redo).
 
-// 8 fp32 -> 3 x 8 bf16.
-__device__ __forceinline__ void split8(const float (&x)[8], uint4 (&out)[3]) {
+// W fp32 (pairs in a word of each piece) -> their three bf16 pieces.
+template <int W>
+__device__ __forceinline__ void split_pieces(const float (&x)[W], uint32_t (&out)[3][W / 2]) {
   typedef __bf16 bf16x2_t __attribute__((__vector_size__(4)));
-  uint32_t w[3][4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < W / 2; ++i) {
     float a = x[2 * i], b = x[2 * i + 1];
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
       const bf16x2_t v = {(__bf16)a, (__bf16)b};
-      w[p][i] = __builtin_bit_cast(uint32_t, v);
-      a -= __uint_as_float(w[p][i] << 16);
-      b -= __uint_as_float(w[p][i] & 0xffff0000u);
+      out[p][i] = __builtin_bit_cast(uint32_t, v);
+      a -= __uint_as_float(out[p][i] << 16);
+      b -= __uint_as_float(out[p][i] & 0xffff0000u);
     }
   }
+}
+
+// 8 fp32 -> 3 x 8 bf16, MFMA operands.
+__device__ __forceinline__ void split8(const float (&x)[8], uint4 (&out)[3]) {
+  uint32_t w[3][4];
+  split_pieces<8>(x, w);
 #pragma unroll
   for (int p = 0; p < 3; ++p) out[p] = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
 }
@@ -1259,52 +1265,36 @@ __device__ __forceinline__ void split_redo(const float* feats, const float* w,
     if (acc[e] * 0.f != 0.f) acc[e] = again[e];
 }
 
-// weight (rows, Ci) fp32 -> (rows, Ci / 16, 3, 16) bf16; thread = 8 consecutive inputs.
-constexpr int kSplitThreads = 256;
-__global__ void __launch_bounds__(kSplitThreads)
-    split_weights_kernel(const float* __restrict__ weight, int64_t n8, uint4* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * kSplitThreads + threadIdx.x;
-  if (i >= n8) return;
-  const float4 u = ((const float4*)weight)[2 * i], v = ((const float4*)weight)[2 * i + 1];
-  const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-  uint4 p[3];
-  split8(x, p);
-#pragma unroll
-  for (int k = 0; k < 3; ++k) out[(i >> 1) * 6 + 2 * k + (i & 1)] = p[k];
-}
-
 // LDS swizzle of a split weight row (6 pieces of 16 bytes): 16 consecutive lanes read one piece of
 // 16 consecutive rows, which without it start in 8 of the 16 bank groups.
 __device__ __forceinline__ int swz_split(int row, int part) { return part ^ ((row >> 3) & 1); }
 
 // WM waves of 32 rows x 32 FN columns.  A row is used by one wave only, so its inputs go from
-// memory to that wave's registers, AHEAD chunks of 16 inputs early, and are split there; the
-// weights of the tap's chunk come into an LDS ring as in conv_mfma_kernel, already split
-// (WSPLIT: by split_weights_kernel) or split by every wave, with the same results, where there is
-// no buffer for that.  Only weights pass through LDS, so four blocks share a CU and their loads,
-// splits and MFMAs overlap: with the rows in the ring as well (two blocks) the three added up.
-// Loads are unconditional (past the end: the last weights again, zero rows): with branches
-// around them the compiler waits for every load in flight before the first use of a row.
-// Bound: the bf16 matrix rate at what the chip's power allows (800 of the 1300 TFLOP/s that a
-// large bf16 product reaches here, with 12-67 % more taps than the rows have).  Against the
-// fp32 MFMA ring kernel this replaced: 32->64 on 1.5 M voxels 745 -> 582 us, 64->64 on 300 k
-// 466 -> 340, 64->64 on 25 k 73 -> 61, 128->256 on 40 k 588 -> 410, 512->512 on 10 k 1494 -> 871.
-// Splitting the next chunk's rows beside the MFMAs: 1-5 % slower.  32 x 128 per wave: 300->288 us
-// to 871->923 as the tiles fill the CUs.
-template <int WM, int FN, int STAGES, int AHEAD, bool WSPLIT, int EPI>
+// memory to that wave's registers, AHEAD chunks of 16 inputs early, and are split there.  The
+// weights are used by all waves: each splits its share of a chunk and writes the pieces into one of
+// two LDS buffers, a chunk early, loaded as long before as the rows.  No buffer outside the
+// block and no second launch: split beforehand in device memory, they would be state between
+// two launches.  Only weights pass through LDS, so four blocks share a CU and their loads, splits
+// and MFMAs overlap.  Loads are unconditional (past the end: the last weights again, zero
+// rows): with branches around them the compiler waits for every load in flight before the first use
+// of a row.
+// Bound: the bf16 matrix rate at what the chip's power allows, with 12-67 % more taps than the rows
+// have.  us, fp32 MFMA ring kernel / weights split beforehand in device memory / this: 32->64 on
+// 1.5 M voxels 788 / 597 / 539, 64->64 on 300 k 478 / 330 / 300, 512->512 on 10 k
+// 1519 / 921 / 814.
+template <int WM, int FN, int AHEAD, int EPI>
 __global__ void __launch_bounds__(64 * WM, WM * FN == 8 ? 4 : 1)
     conv_split_kernel(const float* __restrict__ feats, const float* __restrict__ weight,
-                      const uint4* __restrict__ wsplit, const float* __restrict__ bias,
-                      const int32_t* __restrict__ nbr, const int32_t* __restrict__ order,
-                      int64_t N, int32_t Ci, int32_t Co, int32_t m_tiles, int32_t n_tiles,
-                      int32_t per_xcd, const float* residual, float* out) {
+                      const float* __restrict__ bias, const int32_t* __restrict__ nbr,
+                      const int32_t* __restrict__ order, int64_t N, int32_t Ci, int32_t Co,
+                      int32_t m_tiles, int32_t n_tiles, int32_t per_xcd, const float* residual,
+                      float* out) {
   constexpr int BM = 32 * WM, BN = 32 * FN, NT = 64 * WM;
-  constexpr int PPRB = WSPLIT ? 6 : 4;       // 16-byte pieces per weight row and chunk
-  constexpr int SB = BN * PPRB * 16;         // bytes per stage
-  constexpr int PPW = BN * PPRB / WM;        // pieces per wave
-  constexpr int IPW = (PPW + 63) / 64;       // loads per wave
-  static_assert(BN * PPRB % WM == 0, "every wave issues the same loads");
-  __shared__ __attribute__((aligned(16))) unsigned char ring[STAGES * SB];
+  constexpr int WF = BN * 16 / NT;    // weights per thread and chunk
+  constexpr int ROWB = 3 * 32;        // bytes of a column's chunk, split
+  static_assert(AHEAD % 2 == 0, "buffer parity");
+  static_assert(WF == 2 || WF == 4 || WF == 8, "one load, one write per piece");
+  __shared__ __attribute__((aligned(16))) unsigned char sW[2][BN * ROWB];
   __shared__ int32_t sNbr[BM * kTaps];
   __shared__ int32_t sRow[BM];
   __shared__ uint32_t sMask;
@@ -1346,9 +1336,7 @@ __global__ void __launch_bounds__(64 * WM, WM * FN == 8 ? 4 : 1)
       ak = 0;
       int32_t src = -1;
       if (am) {
-        src = lds_read_i32(sNbr + myrow * kTaps + (__ffs(am) - 1));
-        lds_wait_all();
-        pin(src);
+        src = sNbr[myrow * kTaps + (__ffs(am) - 1)];
         am &= am - 1;
       }
       ap = (src >= 0 ? feats + (int64_t)src * Ci : (const float*)g_zero) + 8 * hf;
@@ -1357,25 +1345,24 @@ __global__ void __launch_bounds__(64 * WM, WM * FN == 8 ? 4 : 1)
     x[0] = u.x; x[1] = u.y; x[2] = u.z; x[3] = u.w;
     x[4] = v.x; x[5] = v.y; x[6] = v.z; x[7] = v.w;
   };
-  // Weight loads into ring stage bstage; past the last chunk the last one again.
+  // Weight loads: inputs wk .. wk + WF - 1 of a chunk's 16, of column wr; past the last chunk the
+  // last one again.
+  const int wr = tid * WF / 16, wk = tid * WF % 16;
+  const float* const wbase = weight + (int64_t)(n0 + wr) * kTaps * Ci + wk;
   uint32_t bm = mask;
-  int bk = 0, bv = mask ? __ffs(mask) - 1 : 0, bstage = 0;
-  uint32_t boff[IPW];
+  int bk = 0, bv = mask ? __ffs(mask) - 1 : 0;
+  auto load_w = [&](float (&w)[WF]) {
+    const float* p = wbase + (bv * Ci + bk * 16);
+    if constexpr (WF == 2) {
+      const float2 u = *(const float2*)p;
+      w[0] = u.x; w[1] = u.y;
+    } else {
 #pragma unroll
-  for (int j = 0; j < IPW; ++j) {
-    const int L = min(wid * PPW + j * 64 + lane, BN * PPRB - 1), r = L / PPRB, pc = L % PPRB;
-    boff[j] = (uint32_t)r * kTaps * cpt * (PPRB * 16) +
-              (WSPLIT ? swz_split(r, pc) : swz<4>(r, pc)) * 16;
-  }
-  const char* const bbase = (WSPLIT ? (const char*)wsplit : (const char*)weight) +
-                            (int64_t)n0 * kTaps * cpt * (PPRB * 16);
-  auto load_b = [&]() {
-    const char* base = bbase + (int64_t)(bv * cpt + bk) * (PPRB * 16);
-#pragma unroll
-    for (int j = 0; j < IPW; ++j)
-      if (PPW % 64 == 0 || j * 64 + lane < PPW)
-        lds_dma16(base + boff[j], (lds_ptr_t)(ring + bstage * SB + (wid * PPW + j * 64) * 16));
-    bstage = bstage + 1 == STAGES ? 0 : bstage + 1;
+      for (int i = 0; i < WF; i += 4) {
+        const float4 u = *(const float4*)(p + i);
+        w[i] = u.x; w[i + 1] = u.y; w[i + 2] = u.z; w[i + 3] = u.w;
+      }
+    }
     if (bk + 1 < cpt) {
       ++bk;
     } else if (bm & (bm - 1)) {
@@ -1384,64 +1371,56 @@ __global__ void __launch_bounds__(64 * WM, WM * FN == 8 ? 4 : 1)
       bk = 0;
     }
   };
+  auto store_w = [&](int buf, const float (&w)[WF]) {
+    uint32_t o[3][WF / 2];
+    split_pieces<WF>(w, o);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      unsigned char* d =
+          sW[buf] + wr * ROWB + swz_split(wr, 2 * p + (wk >> 3)) * 16 + (wk & 7) * 2;
+      if constexpr (WF == 2) *(uint32_t*)d = o[p][0];
+      if constexpr (WF == 4) *(uint2*)d = make_uint2(o[p][0], o[p][1]);
+      if constexpr (WF == 8) *(uint4*)d = make_uint4(o[p][0], o[p][1], o[p][2], o[p][3]);
+    }
+  };
 
-  const uint32_t ring0 = lds_addr(ring);
-  int rstage = 0;
-  auto step = [&](float (&x)[8]) {
-    // This wave's part of the chunk is in LDS: at most the loads of the STAGES - 2 chunks after it
-    // are in flight (row loads in flight only make the wait longer).  After the barrier
-    // every wave's is, and every wave has read the stage that load_b refills.
-    wait_vmcnt<IPW * (STAGES - 2)>();
-    TSC_COMPILER_BARRIER();
+  float x[AHEAD][8], w[AHEAD][WF];
+  auto step = [&](int i) {
+    // After the barrier every wave's part of this chunk is in LDS, and every wave has read the
+    // buffer that the next chunk's weights go to.
+    lds_wait_all();
     __builtin_amdgcn_s_barrier();
     TSC_COMPILER_BARRIER();
-    uint4 as[3];
-    split8(x, as);
-    load_a(x);
-    load_b();
-    const uint32_t b0 = ring0 + rstage * SB;
-    rstage = rstage + 1 == STAGES ? 0 : rstage + 1;
-    constexpr int NP = WSPLIT ? 3 : 2;
-    u32x4 br[FN][NP];
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int r = j * 32 + l32;
-#pragma unroll
-      for (int p = 0; p < NP; ++p)
-        br[j][p] = lds_read16(b0 + (r * PPRB + (WSPLIT ? swz_split(r, 2 * p + hf)
-                                                       : swz<4>(r, 2 * hf + p))) * 16);
-    }
-    lds_wait_all();
     uint4 bs[FN][3];
 #pragma unroll
-    for (int j = 0; j < FN; ++j) {
+    for (int j = 0; j < FN; ++j)
 #pragma unroll
-      for (int p = 0; p < NP; ++p) pin(br[j][p]);
-      if constexpr (WSPLIT) {
-#pragma unroll
-        for (int p = 0; p < 3; ++p) bs[j][p] = __builtin_bit_cast(uint4, br[j][p]);
-      } else {
-        float w[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) w[e] = __uint_as_float(br[j][e >> 2][e & 3]);
-        split8(w, bs[j]);
+      for (int p = 0; p < 3; ++p) {
+        const int r = j * 32 + l32;
+        bs[j][p] = *(const uint4*)(sW[i & 1] + r * ROWB + swz_split(r, 2 * p + hf) * 16);
       }
-    }
+    uint4 as[3];
+    split8(x[i], as);
+    load_a(x[i]);
     split_mma<FN>(as, bs, acc);
+    const int n = (i + 1) % AHEAD;
+    store_w(n & 1, w[n]);
+    load_w(w[n]);
   };
 
   if (nchunks > 0) {
-    float x[AHEAD][8];
 #pragma unroll
-    for (int i = 0; i < AHEAD; ++i) load_a(x[i]);
-#pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s) load_b();
+    for (int i = 0; i < AHEAD; ++i) {
+      load_a(x[i]);
+      load_w(w[i]);
+    }
+    store_w(0, w[0]);
+    load_w(w[0]);
     for (int c = 0; c < nchunks; c += AHEAD) {
 #pragma unroll
-      for (int i = 0; i < AHEAD; ++i) step(x[i]);
+      for (int i = 0; i < AHEAD; ++i) step(i);
     }
   }
-  wait_vmcnt<0>();  // weight loads past the end still write LDS
 
   const int col = n0 + l32;
   if (split_bad<FN>(acc)) {  // wave-uniform
@@ -1484,48 +1463,18 @@ inline bool split_shape(const ConvArgs& a) {
          !(a.Ci == 32 && a.Co == 32);
 }
 
-// Weights split beforehand, or without a buffer for them (calls that may not allocate, captured
-// calls, whose graph would keep the address, more than kSplitMaxBytes, and a failed allocation)
-// in the kernel: the same results.
-constexpr int64_t kSplitMaxBytes = (int64_t)256 << 20;
-
-template <int WM, int FN, int STAGES, int AHEAD, int EPI>
+template <int WM, int FN, int AHEAD, int EPI>
 int launch_split(tsc_ctx* ctx, const ConvArgs& a) {
-  void* buf = nullptr;
-  const int64_t n8 = (int64_t)a.Co * kTaps * a.Ci / 8;
-  bool wsplit = !a.sched_scratch && n8 * 48 <= kSplitMaxBytes;
-  if (wsplit) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) {
-      (void)hipGetLastError();
-      cap = hipStreamCaptureStatusActive;
-    }
-    wsplit = cap == hipStreamCaptureStatusNone &&
-             split_workspace(ctx, (size_t)n8 * 48, &buf) == TSC_OK;
-  }
-  if (wsplit) {
-    ProfScope p(ctx, "conv_split_weights");
-    split_weights_kernel<<<(unsigned)((n8 + kSplitThreads - 1) / kSplitThreads), kSplitThreads, 0,
-                           ctx->stream>>>((const float*)a.weight, n8, (uint4*)buf);
-  }
   const int32_t m_tiles = (int32_t)((a.N + 32 * WM - 1) / (32 * WM));
   const int32_t n_tiles = a.Co / (32 * FN);
   const int32_t per_xcd = tile_grid_per_xcd(m_tiles, n_tiles);
-  static const std::string base = "conv_split_kernel<" + std::to_string(32 * WM) + "x" +
-                                  std::to_string(32 * FN);
-  static const std::string names[2] = {
-      base + ",ab" + (EPI == TSC_EPI_BIAS_RESIDUAL ? ",res>" : ">"),
-      base + (EPI == TSC_EPI_BIAS_RESIDUAL ? ",res>" : ">")};
-  ProfScope p(ctx, names[wsplit].c_str());
-  auto run = [&](auto ws) {
-    conv_split_kernel<WM, FN, STAGES, AHEAD, decltype(ws)::value, EPI>
-        <<<(unsigned)per_xcd * 8u, 64 * WM, 0, ctx->stream>>>(
-            (const float*)a.feats, (const float*)a.weight, (const uint4*)buf,
-            (const float*)a.bias, a.nbr, a.order, a.N, a.Ci, a.Co, m_tiles, n_tiles, per_xcd,
-            (const float*)a.residual, (float*)a.out);
-  };
-  if (wsplit) run(std::true_type());
-  else run(std::false_type());
+  static const std::string name = "conv_split_kernel<" + std::to_string(32 * WM) + "x" +
+                                  std::to_string(32 * FN) +
+                                  (EPI == TSC_EPI_BIAS_RESIDUAL ? ",res>" : ">");
+  ProfScope p(ctx, name.c_str());
+  conv_split_kernel<WM, FN, AHEAD, EPI><<<(unsigned)per_xcd * 8u, 64 * WM, 0, ctx->stream>>>(
+      (const float*)a.feats, (const float*)a.weight, (const float*)a.bias, a.nbr, a.order, a.N,
+      a.Ci, a.Co, m_tiles, n_tiles, per_xcd, (const float*)a.residual, (float*)a.out);
   return check_hip(hipGetLastError(), "conv launch");
 }
 
@@ -1881,15 +1830,14 @@ int dispatch_tiles(tsc_ctx* ctx, const ConvArgs& a) {
     if (a.Co % 64 == 0) return launch_cfg<T, 128, 64, 32, 4, 1, EPI>(ctx, a);
   } else {
     if (split_shape(a)) {
-      if (a.Co % 64 != 0) return launch_split<4, 1, 4, 2, EPI>(ctx, a);
+      if (a.Co % 64 != 0) return launch_split<4, 1, 2, EPI>(ctx, a);
       // Fewer 128 x 64 tiles than CUs (e.g. 25 k voxels of 64 channels): 64 x 64 tiles, or still
       // fewer than CUs, 64 x 32, each with a deeper pipeline, since few blocks share a CU.
-      // 64->64: 25 k voxels 77 / 67 / 75 us in 128 x 64 / 64 x 64 / 64 x 32 tiles, 3 k 61 / 60 / 50.
       const int64_t n64 = a.Co / 64;
       if ((a.N + 127) / 128 * n64 < 256)
-        return (a.N + 63) / 64 * n64 < 256 ? launch_split<2, 1, 8, 4, EPI>(ctx, a)
-                                           : launch_split<2, 2, 8, 4, EPI>(ctx, a);
-      return launch_split<4, 2, 4, 2, EPI>(ctx, a);
+        return (a.N + 63) / 64 * n64 < 256 ? launch_split<2, 1, 4, EPI>(ctx, a)
+                                           : launch_split<2, 2, 4, EPI>(ctx, a);
+      return launch_split<4, 2, 2, EPI>(ctx, a);
     }
     return launch_cfg<T, 128, 32, 32, 4, 1, EPI>(ctx, a);
   }

@@ -52,8 +52,6 @@ struct tsc_ctx {
   void* blaslt = nullptr;
   void* ws_blas = nullptr;
   size_t ws_blas_bytes = 0;
-  void* ws_split = nullptr;    // an fp32 conv's weights, split (conv.hip)
-  size_t ws_split_bytes = 0;
   void* blas_algos = nullptr;  // tuned algorithm per linear shape (linear.hip)
   // Pinned host chunks (and their last copies' events) of the safetensors reader.
   void* st_pin[2] = {nullptr, nullptr};
@@ -78,8 +76,6 @@ int check_hip(hipError_t e, const char* what);
 int workspace(tsc_ctx* ctx, size_t bytes, void** out);
 // The same for ctx->ws_blas.
 int blas_workspace(tsc_ctx* ctx, size_t bytes, void** out);
-// The same for ctx->ws_split (a conv may run while ctx->ws holds its input rows).
-int split_workspace(tsc_ctx* ctx, size_t bytes, void** out);
 // The cached tile schedule of (nbr, order, N, bm).  On a hit *entry->valid is true and
 // entry->buf holds it; on a miss the least recently used entry (at most kSchedCacheEntries) is
 // re-keyed with valid = false and its buffer grown to `bytes`; the caller launches the schedule
