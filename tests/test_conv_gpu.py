@@ -463,10 +463,10 @@ def _conv64(f, w, b, nbr):
 
 
 @pytest.mark.parametrize("n,ci,co", [
-    (1, 32, 64), (31, 48, 64), (65, 64, 64), (3000, 64, 128),        # 64 x 32 tiles
-    (16385, 48, 64), (20001, 32, 64),                                # 64 x 64
-    (32641, 32, 64), (33000, 80, 64), (40003, 64, 128),              # 128 x 64
-    (1, 32, 32 * 3), (127, 64, 32), (129, 48, 96), (5000, 128, 32)]) # 128 x 32
+    (1, 32, 64), (31, 48, 64), (65, 64, 64), (3000, 64, 128),        # 128 x 32 tiles
+    (16385, 48, 64), (20001, 32, 64), (32641, 32, 64), (4096, 64, 512),
+    (1, 32, 32 * 3), (127, 64, 32), (129, 48, 96), (5000, 128, 32),
+    (32769, 32, 64), (33000, 80, 64), (40003, 64, 128), (4097, 64, 512)])  # 128 x 64
 def test_conv_fp32_split_tiles(pkg, dev, n, ci, co):
     """fp32 convs on bf16 pieces, at the edges of every tile and with odd chunk counts per tap.  At
     most 27 Ci products are summed in fp32, each sum rounding by at most 2^-24 of its size: 4e-6

@@ -1269,7 +1269,7 @@ __device__ __forceinline__ void split_redo(const float* feats, const float* w,
 // 16 consecutive rows, which without it start in 8 of the 16 bank groups.
 __device__ __forceinline__ int swz_split(int row, int part) { return part ^ ((row >> 3) & 1); }
 
-// WM waves of 32 rows x 32 FN columns.  A row is used by one wave only, so its inputs go from
+// Four waves of 32 rows x 32 FN columns.  A row is used by one wave only, so its inputs go from
 // memory to that wave's registers, AHEAD chunks of 16 inputs early, and are split there.  The
 // weights are used by all waves: each splits its share of a chunk and writes the pieces into one of
 // two LDS buffers, a chunk early, loaded as long before as the rows.  No buffer outside the
@@ -1282,18 +1282,20 @@ __device__ __forceinline__ int swz_split(int row, int part) { return part ^ ((ro
 // have.  us, fp32 MFMA ring kernel / weights split beforehand in device memory / this: 32->64 on
 // 1.5 M voxels 788 / 597 / 539, 64->64 on 300 k 478 / 330 / 300, 512->512 on 10 k
 // 1519 / 921 / 814.
-template <int WM, int FN, int AHEAD, int EPI>
-__global__ void __launch_bounds__(64 * WM, WM * FN == 8 ? 4 : 1)
+constexpr int kSplitBM = 128, kSplitThreads = 256;
+template <int FN, int EPI>
+__global__ void __launch_bounds__(kSplitThreads, FN == 2 ? 4 : 1)
     conv_split_kernel(const float* __restrict__ feats, const float* __restrict__ weight,
                       const float* __restrict__ bias, const int32_t* __restrict__ nbr,
                       const int32_t* __restrict__ order, int64_t N, int32_t Ci, int32_t Co,
                       int32_t m_tiles, int32_t n_tiles, int32_t per_xcd, const float* residual,
                       float* out) {
-  constexpr int BM = 32 * WM, BN = 32 * FN, NT = 64 * WM;
+  constexpr int BM = kSplitBM, BN = 32 * FN, NT = kSplitThreads;
+  constexpr int AHEAD = 2;            // chunks of rows (and weights) in flight; 4: the same times
   constexpr int WF = BN * 16 / NT;    // weights per thread and chunk
   constexpr int ROWB = 3 * 32;        // bytes of a column's chunk, split
   static_assert(AHEAD % 2 == 0, "buffer parity");
-  static_assert(WF == 2 || WF == 4 || WF == 8, "one load, one write per piece");
+  static_assert(WF == 2 || WF == 4, "one load, one write per piece");
   __shared__ __attribute__((aligned(16))) unsigned char sW[2][BN * ROWB];
   __shared__ int32_t sNbr[BM * kTaps];
   __shared__ int32_t sRow[BM];
@@ -1357,11 +1359,8 @@ __global__ void __launch_bounds__(64 * WM, WM * FN == 8 ? 4 : 1)
       const float2 u = *(const float2*)p;
       w[0] = u.x; w[1] = u.y;
     } else {
-#pragma unroll
-      for (int i = 0; i < WF; i += 4) {
-        const float4 u = *(const float4*)(p + i);
-        w[i] = u.x; w[i + 1] = u.y; w[i + 2] = u.z; w[i + 3] = u.w;
-      }
+      const float4 u = *(const float4*)p;
+      w[0] = u.x; w[1] = u.y; w[2] = u.z; w[3] = u.w;
     }
     if (bk + 1 < cpt) {
       ++bk;
@@ -1379,8 +1378,7 @@ __global__ void __launch_bounds__(64 * WM, WM * FN == 8 ? 4 : 1)
       unsigned char* d =
           sW[buf] + wr * ROWB + swz_split(wr, 2 * p + (wk >> 3)) * 16 + (wk & 7) * 2;
       if constexpr (WF == 2) *(uint32_t*)d = o[p][0];
-      if constexpr (WF == 4) *(uint2*)d = make_uint2(o[p][0], o[p][1]);
-      if constexpr (WF == 8) *(uint4*)d = make_uint4(o[p][0], o[p][1], o[p][2], o[p][3]);
+      else *(uint2*)d = make_uint2(o[p][0], o[p][1]);
     }
   };
 
@@ -1463,16 +1461,16 @@ inline bool split_shape(const ConvArgs& a) {
          !(a.Ci == 32 && a.Co == 32);
 }
 
-template <int WM, int FN, int AHEAD, int EPI>
+template <int FN, int EPI>
 int launch_split(tsc_ctx* ctx, const ConvArgs& a) {
-  const int32_t m_tiles = (int32_t)((a.N + 32 * WM - 1) / (32 * WM));
+  const int32_t m_tiles = (int32_t)((a.N + kSplitBM - 1) / kSplitBM);
   const int32_t n_tiles = a.Co / (32 * FN);
   const int32_t per_xcd = tile_grid_per_xcd(m_tiles, n_tiles);
-  static const std::string name = "conv_split_kernel<" + std::to_string(32 * WM) + "x" +
+  static const std::string name = "conv_split_kernel<" + std::to_string(kSplitBM) + "x" +
                                   std::to_string(32 * FN) +
                                   (EPI == TSC_EPI_BIAS_RESIDUAL ? ",res>" : ">");
   ProfScope p(ctx, name.c_str());
-  conv_split_kernel<WM, FN, AHEAD, EPI><<<(unsigned)per_xcd * 8u, 64 * WM, 0, ctx->stream>>>(
+  conv_split_kernel<FN, EPI><<<(unsigned)per_xcd * 8u, kSplitThreads, 0, ctx->stream>>>(
       (const float*)a.feats, (const float*)a.weight, (const float*)a.bias, a.nbr, a.order, a.N,
       a.Ci, a.Co, m_tiles, n_tiles, per_xcd, (const float*)a.residual, (float*)a.out);
   return check_hip(hipGetLastError(), "conv launch");
@@ -1830,14 +1828,18 @@ int dispatch_tiles(tsc_ctx* ctx, const ConvArgs& a) {
     if (a.Co % 64 == 0) return launch_cfg<T, 128, 64, 32, 4, 1, EPI>(ctx, a);
   } else {
     if (split_shape(a)) {
-      if (a.Co % 64 != 0) return launch_split<4, 1, 2, EPI>(ctx, a);
-      // Fewer 128 x 64 tiles than CUs (e.g. 25 k voxels of 64 channels): 64 x 64 tiles, or still
-      // fewer than CUs, 64 x 32, each with a deeper pipeline, since few blocks share a CU.
-      const int64_t n64 = a.Co / 64;
-      if ((a.N + 127) / 128 * n64 < 256)
-        return (a.N + 63) / 64 * n64 < 256 ? launch_split<2, 1, 4, EPI>(ctx, a)
-                                           : launch_split<2, 2, 4, EPI>(ctx, a);
-      return launch_split<4, 2, 2, EPI>(ctx, a);
+      // 128 x 32 tiles while all of them have their place on the chip at once (two blocks per CU):
+      // a tile's time is its chain of chunks, and theirs take less.  Past that 128 x 64, whose
+      // rows are split for twice the columns.  us, fp32 MFMA ring kernel / 128 x 32 / 128 x 64 (tiles
+      // of 128 x 32):
+      //   64->64     7 k voxels    52 / 42 / 63  (110)   30 k   72 / 60 / 65 (470)
+      //   64->64    55 k          125 / 105 / 85 (860)   40 k  122 / 82 / 81 (626)
+      //   256->256   3 k          173 / 148 / 223 (192)   7 k  255 / 213 / 230 (440)
+      //   256->256  10 k          435 / 296 / 282 (632)
+      //   512->512 500            331 / 286 / 482  (64)   3 k  489 / 418 / 490 (384)
+      if (a.Co % 64 != 0 || (a.N + 127) / 128 * (a.Co / 32) <= 512)
+        return launch_split<1, EPI>(ctx, a);
+      return launch_split<2, EPI>(ctx, a);
     }
     return launch_cfg<T, 128, 32, 32, 4, 1, EPI>(ctx, a);
   }
