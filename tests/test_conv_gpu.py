@@ -565,6 +565,63 @@ def test_conv_generic_by_grid_size(pkg, dev, dtype, ci, co, n):
     assert ((out.double() - want).norm() / want.norm()).item() <= tol[dtype]
 
 
+@pytest.mark.parametrize("sx,sw", [(1e-36, 1.0), (1e-37, 1.0), (1e-39, 1e10), (1.0, 1e-36),
+                                   (1e10, 1e-39), (1e-20, 1e-16)])
+@pytest.mark.parametrize("n,ci,co,misaligned", [(300, 32, 64, False), (33000, 48, 64, False),
+                                                (300, 64, 96, True)])
+def test_conv_fp32_split_small_values(pkg, dev, n, ci, co, misaligned, sx, sw):
+    """bf16 ends at 2^-133, so the pieces of values below 2^-110 do not add up to them.  Every other
+    row (and column) is scaled down; sums of such rows alone are as good as any: 4e-6 (see
+    test_conv_fp32_split_tiles; unsplit, rows of 1e-36 would be 3e-5 off, of 1e-37 3e-4), and one unit
+    of the smallest float for each of at most 27 Ci additions.  No result depends on what else is in
+    its tile: the same bits in another order."""
+    print(f"  conv fp32 small N={n} {ci}->{co} {sx} {sw}", flush=True)
+    put = (lambda t: _offset(t)) if misaligned else (lambda t: t)
+    rng = np.random.default_rng(n)
+    nbr = _random_table(n, 11, 0.3)
+    small = np.arange(n) % 3 != 0
+    like = small[nbr] == small[:, None]  # half of the rows have neighbors of their own kind only
+    nbr[(np.arange(n) % 2 == 0)[:, None] & ~like] = -1
+    alone = torch.from_numpy(small & (np.arange(n) % 2 == 0)).to(dev)
+    nbr = torch.from_numpy(nbr).to(dev)
+    f = torch.from_numpy(pkg.workloads.features(n, ci, 1)).to(dev).double()
+    f[torch.from_numpy(small).to(dev)] *= sx
+    f = f.float()
+    w = torch.from_numpy(pkg.workloads.conv_weight(co, ci, 2)).to(dev).double()
+    w[::2] *= sw
+    w = w.float()
+    out = pkg.sparse_conv3d(put(f), put(w), None, nbr)
+    want = _conv64(f, w, torch.zeros(co, device=dev), nbr)
+    tiny = 2.0 ** -149 * 27 * ci
+    for rows in (alone, ~alone):
+        for cols in (slice(0, None, 2), slice(1, None, 2)):
+            err = (out.double() - want)[rows, cols]
+            ref = want[rows, cols]
+            assert err.norm() <= 4e-6 * ref.norm() + tiny * ref.numel() ** 0.5
+    order = torch.from_numpy(rng.permutation(n).astype(np.int32)).to(dev)
+    assert torch.equal(pkg.sparse_conv3d(put(f), put(w), None, nbr, order=order), out)
+    assert torch.equal(pkg.sparse_conv3d(f, w, None, nbr), out)
+
+
+def test_conv_fp32_single_products(pkg, dev):
+    """A sum that is one product (all other inputs zero) is rounded at most three times by 2^-24, and
+    of the nine products of its pieces the three left out come to 2^-24: within 2.5e-7 of it, and
+    3.6e-8 on average (root mean square: 3.4e-8 measured)."""
+    n, ci, co = 20000, 32, 64
+    g = torch.Generator(device=dev).manual_seed(3)
+    f = torch.zeros((n, ci), device=dev)
+    at = torch.randint(0, ci, (n, 1), generator=g, device=dev)
+    f.scatter_(1, at, torch.randn((n, 1), generator=g, device=dev))
+    w = torch.randn((co, 3, 3, 3, ci), generator=g, device=dev)
+    nbr = torch.full((n, 27), -1, dtype=torch.int32, device=dev)
+    nbr[:, 13] = torch.arange(n, device=dev)
+    out = pkg.sparse_conv3d(f, w, None, nbr).double()
+    want = f.double() @ w[:, 1, 1, 1].double().t()
+    err = (out - want).abs() / want.abs()
+    print(f"  conv fp32 single products {err.max():.2e} {err.pow(2).mean().sqrt():.2e}", flush=True)
+    assert err.max() <= 2.5e-7 and err.pow(2).mean().sqrt() <= 3.6e-8
+
+
 def test_conv_fp32_keeps_nothing_in_the_context(pkg, dev):
     """An fp32 conv only enqueues: no device memory is taken (a copy of these weights in bf16 pieces
     would be 170 MB) and nothing is left behind that the next conv on the context could meet."""

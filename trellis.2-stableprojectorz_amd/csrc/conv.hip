@@ -1187,13 +1187,22 @@ int launch_narrow(tsc_ctx* ctx, const ConvArgs& a) {
 //
 // v_mfma_f32_32x32x2_f32 runs at 1/16 of the bf16 rate, so an fp32 product as six bf16 ones is
 // 2.7x as fast.  x = x0 + x1 + x2, each the bf16 nearest to what the ones before left over: 24 bits
-// and both signs, so the sum is x itself (x2 loses bits only where |x| is below 2^-109).  Of the
-// nine products x_i w_j the three with i + j > 2 are left out: each is below 2^-25 of x w, less
-// than the rounding of the sums.  All are summed in fp32 by the MFMAs, of every 16 inputs the
-// smallest first.  Error against fp64 (rel. 2-norm, N(0,1) rows), fp32 MFMAs / this: 64->64
-// 5.9e-7 / 5.0e-7, 128->256 8.2e-7 / 7.1e-7, 512->512 1.7e-6 / 1.5e-6.  An infinite or NaN operand
-// (or one that rounds to an infinite bf16) has no such split; it always leaves an infinite or
-// NaN sum, and those outputs are summed again on fp32 MFMAs (split_redo).
+// and both signs, so for |x| >= 2^-100 the sum is x itself.  Of the nine products x_i w_j the three
+// with i + j > 2 are left out: each is below 2^-25 of x w, less than the rounding of the sums.  All
+// are summed in fp32 by the MFMAs, of every 16 inputs the smallest first.  Error against fp64 (rel.
+// 2-norm, N(0,1) rows), fp32 MFMAs / this: 64->64 5.8e-7 / 5.0e-7, 128->256 8.3e-7 / 7.2e-7,
+// 512->512 1.7e-6 / 1.5e-6; sums of 32 products 1.0e-7 / 6.8e-8; a sum that is one product only
+// (all others zero) 2.5e-8 / 3.4e-8, at most 6.0e-8 / 1.5e-7 (1.2e-7 with two more products).
+//
+// Two kinds of sums are made again on fp32 MFMAs (split_redo):
+//   not finite  An infinite or NaN operand, or one that rounds to an infinite bf16, has no such split;
+//               it always leaves an infinite or NaN sum.
+//   too small   bf16 ends at 2^-133, so pieces of an operand x lose bits below 2^-110 (the third),
+//               2^-117 (the second), 2^-126 (the first): at most 2^-134 of absolute value, which
+//               its partner w multiplies.  With E the sum of |w| over the operands x below 2^-100 and
+//               of |x| over such w, the sum is off by at most E 2^-134: made again where that could
+//               be 2^-28 of it.
+// Either is a property of the sum alone, whatever other rows share its tile.
 
 // W fp32 (pairs in a word of each piece) -> their three bf16 pieces.
 template <int W>
@@ -1232,37 +1241,144 @@ __device__ __forceinline__ void split_mma(const uint4 (&a)[3], const uint4 (&b)[
       for (int j = 0; j < FN; ++j) mfma_piece<__bf16>(a[p], b[j][q - p], acc[j]);
 }
 
-// Whether a sum of this wave is infinite or NaN.
-template <int FN>
-__device__ __forceinline__ bool split_bad(const f32x16_t (&acc)[FN]) {
-  float z = 0.f;
-#pragma unroll
-  for (int j = 0; j < FN; ++j)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) z = fmaf(acc[j][e], 0.f, z);
-  return __any(z != 0.f);  // NaN compares unequal
-}
+// Smallest (nonzero) and largest of the operands a thread has seen.  lo: 2 |x| - 1 as integers, so
+// that a zero comes out as the largest.  asm: one instruction each, and where they are
+// written (the compiler gathers them behind the loop, which keeps all operands alive).
+constexpr uint32_t kSplitSmall = 2 * ((127 - 100) << 23);  // 2^-100
+struct SplitRange {
+  uint32_t lo = ~0u;
+  float hi = 0.f;
+  __device__ __forceinline__ void add(float x, float y) {
+    const uint32_t u = 2u * __float_as_uint(x) - 1u, v = 2u * __float_as_uint(y) - 1u;
+    asm volatile("v_min3_u32 %0, %0, %1, %2" : "+v"(lo) : "v"(u), "v"(v));
+    asm volatile("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(hi) : "v"(x), "v"(y));
+  }
+  __device__ __forceinline__ bool small() const { return lo < kSplitSmall - 1u; }
+};
 
-// The sums that are not finite, again on fp32 operands straight from memory.  nbr27: this lane's
-// row's 27 neighbors; w: this lane's column's 27 rows of Ci weights.
+// The sums that are not finite, and with `small` those that are too small, again on fp32 operands
+// straight from memory.  nbr27: this lane's row's 27 neighbors; w: this lane's column's 27 rows of
+// Ci weights.  E comes from bf16 MFMAs: it is wanted to a few bits.
 __device__ __forceinline__ void split_redo(const float* feats, const float* w,
                                            const int32_t* nbr27, uint32_t taps, int32_t Ci,
-                                           f32x16_t& acc) {
+                                           bool small, f32x16_t& acc) {
   const int hf = (threadIdx.x & 63) >> 5;
-  f32x16_t again;
+  f32x16_t sum, err;
 #pragma unroll
-  for (int e = 0; e < 16; ++e) again[e] = 0.f;
+  for (int e = 0; e < 16; ++e) sum[e] = err[e] = 0.f;
   for (; taps; taps &= taps - 1) {
     const int v = __ffs(taps) - 1;
     const int32_t src = nbr27[v];
-    const float* ap = src >= 0 ? feats + (int64_t)src * Ci : (const float*)g_zero;
-    const float* bp = w + (int64_t)v * Ci;
-    for (int k = hf; k < Ci; k += 2)
-      again = __builtin_amdgcn_mfma_f32_32x32x2f32(ap[k], bp[k], again, 0, 0, 0);
+    const float* ap = (src >= 0 ? feats + (int64_t)src * Ci : (const float*)g_zero) + 8 * hf;
+    const float* bp = w + (int64_t)v * Ci + 8 * hf;
+#pragma unroll 1
+    for (int k = 0; k < Ci; k += 16) {
+      float a[8], b[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        a[i] = ap[k + i];
+        b[i] = bp[k + i];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        sum = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[i], sum, 0, 0, 0);
+      if (small) {  // uniform
+        bf16x8_t at, aa, bt, ba;  // 1 where small, |x|
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          at[i] = (__bf16)(a[i] != 0.f && fabsf(a[i]) < 0x1p-100f ? 1.f : 0.f);
+          bt[i] = (__bf16)(b[i] != 0.f && fabsf(b[i]) < 0x1p-100f ? 1.f : 0.f);
+          aa[i] = (__bf16)fabsf(a[i]);
+          ba[i] = (__bf16)fabsf(b[i]);
+        }
+        err = __builtin_amdgcn_mfma_f32_32x32x16_bf16(at, ba, err, 0, 0, 0);
+        err = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aa, bt, err, 0, 0, 0);
+      }
+    }
   }
 #pragma unroll
   for (int e = 0; e < 16; ++e)
-    if (acc[e] * 0.f != 0.f) acc[e] = again[e];
+    if (acc[e] * 0.f != 0.f || !(fabsf(acc[e]) >= err[e] * 0x1p-106f)) acc[e] = sum[e];
+}
+
+// After the sums: makes those again that the split does not hold for.  live: bit r: row r of the
+// wave exists; hiw: the largest |weight| of this lane's columns; wsmall (uniform): the wave has used
+// a small weight.  A sum can only be too small for its small inputs if it is below 27 Ci hiw 2^-106
+// (c doubles that twice, for the roundings of E and of this): for weights of ordinary size only
+// a sum of zero is, and only then, or after a small weight, the wave looks at its inputs (64->64 on
+// 25 k voxels: 59 us, all inputs zero 97, all of 1e-36 217; the fp32 MFMA kernel took 73).
+template <int FN>
+__device__ __forceinline__ void split_finish(const float* feats, const float* w,
+                                             const int32_t* nbr27, uint32_t taps, int32_t Ci,
+                                             uint32_t live, const float (&hiw)[FN], bool wsmall,
+                                             f32x16_t (&acc)[FN]) {
+  const int hf = (threadIdx.x & 63) >> 5;
+  const float c = (float)(4 * kTaps * Ci) * 0x1p-106f;
+  float least[FN], z = 0.f;
+  bool look = wsmall, redo = false, xsmall = false;
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    least[j] = INFINITY;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      least[j] = fminf(least[j], fabsf(acc[j][e]));
+      z = fmaf(acc[j][e], 0.f, z);  // NaN if a sum is infinite or NaN
+    }
+    look |= least[j] < c * hiw[j];
+  }
+  redo = z != 0.f;
+  if (__any(look) && live != ~0u) {  // without the rows that are not there
+    look = wsmall;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      least[j] = INFINITY;
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (live >> (4 * hf) >> (8 * (e >> 2) + (e & 3)) & 1u)
+          least[j] = fminf(least[j], fabsf(acc[j][e]));
+      look |= least[j] < c * hiw[j];
+    }
+  }
+  if (__any(look)) {
+    uint32_t lo = ~0u;
+    float hix = 0.f;
+    for (uint32_t m = taps; m;) {  // several taps at a time, for loads in flight
+      constexpr int T = 2 * FN;
+      const float* p[T];
+#pragma unroll
+      for (int t = 0; t < T; ++t, m &= m - 1) {
+        const int32_t src = m ? nbr27[__ffs(m) - 1] : -1;
+        p[t] = (src >= 0 ? feats + (int64_t)src * Ci : (const float*)g_zero) + 8 * hf;
+      }
+#pragma unroll FN
+      for (int k = 0; k < Ci; k += 16) {
+        float x[T][8];
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) x[t][i] = p[t][k + i];
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            lo = min(lo, 2u * __float_as_uint(x[t][i]) - 1u);
+            hix = fmaxf(hix, fabsf(x[t][i]));
+          }
+      }
+    }
+    xsmall = __any(lo < kSplitSmall - 1u);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) hix = fmaxf(hix, __shfl_xor(hix, off, 64));
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+      redo |= least[j] < c * ((xsmall ? hiw[j] : 0.f) + (wsmall ? hix : 0.f));
+  }
+  if (__any(redo)) {
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+      split_redo(feats, w + (int64_t)(32 * j) * kTaps * Ci, nbr27, taps, Ci, xsmall || wsmall,
+                 acc[j]);
+  }
 }
 
 // LDS swizzle of a split weight row (6 pieces of 16 bytes): 16 consecutive lanes read one piece of
@@ -1280,8 +1396,9 @@ __device__ __forceinline__ int swz_split(int row, int part) { return part ^ ((ro
 // of a row.
 // Bound: the bf16 matrix rate at what the chip's power allows, with 12-67 % more taps than the rows
 // have.  us, fp32 MFMA ring kernel / weights split beforehand in device memory / this: 32->64 on
-// 1.5 M voxels 788 / 597 / 539, 64->64 on 300 k 478 / 330 / 300, 512->512 on 10 k
-// 1519 / 921 / 814.
+// 1.5 M voxels 788 / 597 / 560, 64->64 on 300 k 478 / 330 / 303, 512->512 on 10 k
+// 1519 / 921 / 820.  Looking for small weights is 1-2 % of that (for small inputs too, in every
+// chunk: 5-16 %).
 constexpr int kSplitBM = 128, kSplitThreads = 256;
 template <int FN, int EPI>
 __global__ void __launch_bounds__(kSplitThreads, FN == 2 ? 4 : 1)
@@ -1300,6 +1417,8 @@ __global__ void __launch_bounds__(kSplitThreads, FN == 2 ? 4 : 1)
   __shared__ int32_t sNbr[BM * kTaps];
   __shared__ int32_t sRow[BM];
   __shared__ uint32_t sMask;
+  __shared__ uint32_t sHi[BN];  // each column's largest |weight|, as its bits
+  __shared__ uint32_t sSmall;   // a weight is small
 
   int m_tile, n_tile;
   if (!tile_of(blockIdx.x, m_tiles, n_tiles, per_xcd, nullptr, &m_tile, &n_tile)) return;
@@ -1307,7 +1426,8 @@ __global__ void __launch_bounds__(kSplitThreads, FN == 2 ? 4 : 1)
   const int n0 = n_tile * BN;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, l32 = lane & 31, hf = lane >> 5;
 
-  if (tid == 0) sMask = 0u;
+  if (tid == 0) sMask = sSmall = 0u;
+  if (tid < BN) sHi[tid] = 0u;
   for (int r = tid; r < BM; r += NT) {
     const int64_t pos = m0 + r;
     sRow[r] = (pos < N) ? (order ? order[pos] : (int32_t)pos) : -1;
@@ -1370,9 +1490,12 @@ __global__ void __launch_bounds__(kSplitThreads, FN == 2 ? 4 : 1)
       bk = 0;
     }
   };
+  SplitRange range;
   auto store_w = [&](int buf, const float (&w)[WF]) {
     uint32_t o[3][WF / 2];
     split_pieces<WF>(w, o);
+#pragma unroll
+    for (int i = 0; i < WF; i += 2) range.add(w[i], w[i + 1]);
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
       unsigned char* d =
@@ -1420,13 +1543,17 @@ __global__ void __launch_bounds__(kSplitThreads, FN == 2 ? 4 : 1)
     }
   }
 
+  // The weights that a wave has used were split by all four.
+  atomicMax(&sHi[wr], __float_as_uint(range.hi));
+  if (range.small()) sSmall = 1u;
+  __syncthreads();
   const int col = n0 + l32;
-  if (split_bad<FN>(acc)) {  // wave-uniform
+  float hiw[FN];
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
-      split_redo(feats, weight + (int64_t)(col + 32 * j) * kTaps * Ci, sNbr + myrow * kTaps, mask,
-                 Ci, acc[j]);
-  }
+  for (int j = 0; j < FN; ++j) hiw[j] = __uint_as_float(sHi[32 * j + l32]);
+  split_finish<FN>(feats, weight + (int64_t)col * kTaps * Ci, sNbr + myrow * kTaps, mask, Ci,
+                   (uint32_t)__ballot(sRow[myrow] >= 0), hiw,
+                   __builtin_amdgcn_readfirstlane(sSmall) != 0u, acc);
 
   // A store writes 32 consecutive columns of two rows.  Residual values first: all loads before
   // the first store (an output may alias the residual element by element).
@@ -1557,11 +1684,12 @@ __global__ void __launch_bounds__(kGenThreads)
   };
   const int part = lane >> 5;
   const int ar = wm * 32 + (lane & 31), br = wn * 32 + (lane & 31);
+  SplitRange range;  // of this lane's column's weights
   auto compute = [&](int buf) {
     if constexpr (SPLIT) {
       uint4 as[3], bs[1][3];
+      float x[8];
       auto split_row = [&](const unsigned char* row, int r, uint4(&o)[3]) {
-        float x[8];
 #pragma unroll
         for (int k = 0; k < 2; ++k)
           *(float4*)(x + 4 * k) = *(const float4*)(row + r * KB + swz<4>(r, 2 * part + k) * 16);
@@ -1569,6 +1697,8 @@ __global__ void __launch_bounds__(kGenThreads)
       };
       split_row(sA[buf], ar, as);
       split_row(sB[buf], br, bs[0]);
+#pragma unroll
+      for (int i = 0; i < 8; i += 2) range.add(x[i], x[i + 1]);
       split_mma<1>(as, bs, *(f32x16_t(*)[1])&acc);
     } else {
       const uint4 a = *(const uint4*)(&sA[buf][ar * KB + swz<2>(ar, part) * 16]);
@@ -1701,9 +1831,10 @@ __global__ void __launch_bounds__(kGenThreads)
   const int co = n0 + wn * 32 + (lane & 31);
   if (co >= Co) return;
   if constexpr (SPLIT) {
-    if (split_bad<1>(*(const f32x16_t(*)[1])&acc))
-      split_redo((const float*)feats, (const float*)weight + (int64_t)co * kTaps * Ci,
-                 sNbr + ar * kTaps, mask, Ci, acc);
+    const float hiw[1] = {fmaxf(range.hi, __shfl_xor(range.hi, 32, 64))};
+    split_finish<1>((const float*)feats, (const float*)weight + (int64_t)co * kTaps * Ci,
+                    sNbr + ar * kTaps, mask, Ci, (uint32_t)__ballot(sRow[ar] >= 0), hiw,
+                    __any(range.small()), *(f32x16_t(*)[1])&acc);
   }
   const float bv = bias ? to_f32<T>(bias[co]) : 0.f;
   // Residual values first, all loads before the first store (see conv_regstage_kernel).
