@@ -128,6 +128,29 @@ def test_map_near_sorted_input(pkg, dev, order):
     _check(m, coords, 1, (512, 512, 512), (1, 1, 1))
 
 
+@pytest.mark.parametrize("n,batch", [(1177600, 1), (1177601, 1), (614400, 2), (614401, 2)])
+@pytest.mark.parametrize("shuffle", [False, True])
+def test_map_bucket_block_sizes(pkg, dev, n, batch, shuffle):
+    """Either side of the sizes at which the bucket blocks grow, for bucket ranges inside the LDS bitmap
+    (one sample) and past it (two): buckets of a few hundred voxels, one of 4096 and some of
+    30000.  Every output equals the bitmap build's (which the other tests hold to the oracle)."""
+    cells = batch << 27
+    third = n // 3
+    runs = [np.arange(4096), (1 << 19) + 4 * np.arange(third)]
+    left = n - 4096 - third
+    runs.append((1 << 22) + np.arange(left) * ((cells - (1 << 22)) // left))
+    key = np.concatenate(runs).astype(np.int64)
+    assert len(np.unique(key)) == n and key.max() < cells
+    if shuffle:
+        key = np.random.default_rng(n).permutation(key)
+    coords = np.stack([key >> 27, key >> 18 & 511, key >> 9 & 511, key & 511], axis=1).astype(np.int32)
+    shape = (512, 512, 512)
+    got = _build(pkg, dev, coords, batch, shape, method="radix")
+    want = _build(pkg, dev, coords, batch, shape, method="bitmap")
+    assert torch.equal(got.nbr, want.nbr)
+    assert torch.equal(got.keys, want.keys) and torch.equal(got.perm, want.perm)
+
+
 @pytest.mark.parametrize("method", METHODS)
 def test_map_bucket_over_65536(pkg, dev, method):
     """A dense 256x512 half slice of 512^3 is one 2^17-cell key bucket of 131072 voxels: past the

@@ -27,16 +27,12 @@
 namespace tsc {
 namespace {
 
-constexpr int RT = 512;             // threads per block (256 x 16: the 1.5 M voxel map, whose
-                                    // largest bucket holds 8144, 113 us against 104)
-constexpr int RI = 8;               // items per thread
-constexpr int RTILE = RT * RI;      // elements per tile
-constexpr int WAVES = RT / 64;
+constexpr int RTILE = 4096;         // elements a bucket block holds in registers
+constexpr int ST = 256;             // threads per block of the scan over tiles
 constexpr int TBMAX = 10;           // bucket digit bits
 constexpr int NBMAX = 1 << TBMAX;   // buckets
 constexpr int LBITS = 9;            // local pass digit bits
 constexpr int LNB = 1 << LBITS;
-constexpr int LPT = LNB / RT;       // local digits owned per thread
 constexpr int PT = 1024;            // pack / partition threads per block
 constexpr int PI = 8;               // pack / partition items per thread (512 x 16: Morton pack
                                     // 19.6 -> 14.7 us at 1.5 M voxels, the others equal)
@@ -147,7 +143,7 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
 }
 
 // Exclusive scan of v over the block's NW waves; *total receives the block sum.
-template <int NW = WAVES>
+template <int NW>
 __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int* total) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int incl = wave_incl_scan(v);
@@ -167,30 +163,30 @@ __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int* total) {
 // Block d: exclusive scan over tiles of bucket d's counts (in place) and totals[d] = its sum.
 // Block 0 also sets the status word from the pack kernel's out-of-range tile flags (the fill
 // adds the duplicate bit later in stream order).
-__global__ void __launch_bounds__(RT)
+__global__ void __launch_bounds__(ST)
     scan_kernel(int* __restrict__ counts, int ntiles, int* __restrict__ totals,
                 const int* __restrict__ oob_tile, uint32_t* __restrict__ status) {
-  __shared__ int wsum[WAVES];
+  __shared__ int wsum[ST / 64];
   int* c = counts + (int64_t)blockIdx.x * ntiles;
   int carry = 0;
-  for (int base = 0; base < ntiles; base += RT) {
+  for (int base = 0; base < ntiles; base += ST) {
     const int i = base + threadIdx.x;
     const int v = (i < ntiles) ? c[i] : 0;
     int tot;
-    const int pre = block_excl_scan(v, wsum, &tot);
+    const int pre = block_excl_scan<ST / 64>(v, wsum, &tot);
     if (i < ntiles) c[i] = carry + pre;
     carry += tot;
   }
   if (threadIdx.x == 0) totals[blockIdx.x] = carry;
   if (blockIdx.x == 0) {
     int any = 0;
-    for (int i = threadIdx.x; i < ntiles; i += RT) any |= oob_tile[i];
+    for (int i = threadIdx.x; i < ntiles; i += ST) any |= oob_tile[i];
     any = __syncthreads_or(any);
     if (threadIdx.x == 0) status[0] = any ? (uint32_t)TSC_MAP_OUT_OF_RANGE : 0u;
   }
 }
 
-// Stable ranks of one wave's RI items (lanes = consecutive elements, items in order) among equal
+// Stable ranks of one wave's N_ITEMS items (lanes = consecutive elements, items in order) among equal
 // digits: peers = lanes with the same digit (one ballot per digit bit), rank = popcount of the
 // lower peers + the wave's running count of that digit (cnt, in LDS, advanced by the first peer).
 template <typename K, int N_ITEMS>
@@ -401,8 +397,10 @@ __device__ __forceinline__ int64_t lower_bound(const K* keys, int64_t lo, int64_
   return lo;
 }
 
-// Exclusive scan of the LNB-bin histogram in run[] (in place), LPT bins per thread.
+// Exclusive scan of the LNB-bin histogram in run[] (in place) by RT threads.
+template <int RT>
 __device__ __forceinline__ void scan_bins(int* run, int* wsum) {
+  constexpr int LPT = LNB / RT;
   const int tid = threadIdx.x;
   int c[LPT], sum = 0;
 #pragma unroll
@@ -411,7 +409,7 @@ __device__ __forceinline__ void scan_bins(int* run, int* wsum) {
     sum += c[q];
   }
   int tot;
-  int pre = block_excl_scan(sum, wsum, &tot);
+  int pre = block_excl_scan<RT / 64>(sum, wsum, &tot);
 #pragma unroll
   for (int q = 0; q < LPT; ++q) {
     run[tid * LPT + q] = pre;
@@ -420,8 +418,10 @@ __device__ __forceinline__ void scan_bins(int* run, int* wsum) {
 }
 
 // wcnt[w][d] (each wave's count of digit d) -> each wave's exclusive offset among the waves;
-// returns the per-thread totals of its LPT digits in cnt.
-__device__ __forceinline__ void wave_offsets(int (*wcnt)[LNB], int (&cnt)[LPT]) {
+// returns the per-thread totals of its digits (RT threads) in cnt.
+template <int RT>
+__device__ __forceinline__ void wave_offsets(int (*wcnt)[LNB], int (&cnt)[LNB / RT]) {
+  constexpr int LPT = LNB / RT, WAVES = RT / 64;
   const int tid = threadIdx.x;
 #pragma unroll
   for (int q = 0; q < LPT; ++q) {
@@ -466,13 +466,16 @@ struct GatherSrc {
   uint32_t* status;
 };
 
-template <typename K>
+template <typename K, int RT>
 __global__ void __launch_bounds__(RT)
     bucket_sort_kernel(K* k0, int32_t* v0, K* k1, int32_t* v1, K* __restrict__ kout,
                        int32_t* __restrict__ vout, const int* __restrict__ totals,
                        const int* __restrict__ bstart, int nbk,
                        int lb, int64_t cells, int64_t Z, int64_t ncol, int64_t n,
                        int32_t* __restrict__ col_start, GatherSrc<K> gs) {
+  constexpr int RI = RTILE / RT;  // items per thread
+  constexpr int WAVES = RT / 64;
+  constexpr int LPT = LNB / RT;   // local digits owned per thread
   // smem: the key bitmap, or the LSD digit counters run[LNB] + wcnt[WAVES][LNB]; before either,
   // the gather pipeline's expanded source positions of the bucket's elements.
   __shared__ __attribute__((aligned(16))) uint32_t
@@ -516,12 +519,12 @@ __global__ void __launch_bounds__(RT)
         rl[k] = gs.toff[(int64_t)t * (nbk + 1) + b + 1] - ra[k];
       }
       int tot;
-      rb0[k] = carry + block_excl_scan(rl[k], wsum, &tot);
+      rb0[k] = carry + block_excl_scan<WAVES>(rl[k], wsum, &tot);
       carry += tot;
       below += ra[k];
     }
     int tot_below;
-    (void)block_excl_scan(below, wsum, &tot_below);  // elements of smaller digits: the start
+    (void)block_excl_scan<WAVES>(below, wsum, &tot_below);  // elements of smaller digits: the start
     start = tot_below;
     size = carry;
     if (b == 0 && gs.status) {
@@ -661,7 +664,7 @@ __global__ void __launch_bounds__(RT)
 #pragma unroll
       for (int q = 0; q < kWpt; ++q) sum += cw[q];
       int tot;
-      int pre = block_excl_scan(sum, wsum, &tot);
+      int pre = block_excl_scan<WAVES>(sum, wsum, &tot);
       if (wpt == kWpt) {
         uint32_t pk[kWpt / 2];
 #pragma unroll
@@ -780,7 +783,7 @@ __global__ void __launch_bounds__(RT)
       for (int i = tid; i < size; i += RT)
         atomicAdd(&run[digit_of<K>(ks[start + i], shift, mask)], 1);
       __syncthreads();
-      scan_bins(run, wsum);
+      scan_bins<RT>(run, wsum);
       for (int c0 = 0; c0 < size; c0 += RTILE) {
         for (int i = tid; i < WAVES * LNB; i += RT) (&wcnt[0][0])[i] = 0;
         __syncthreads();
@@ -799,7 +802,7 @@ __global__ void __launch_bounds__(RT)
         wave_rank<K, RI>(kk, wfirst, wlimit, shift, dbits, wcnt[w], lr);
         __syncthreads();
         int cnt[LPT];
-        wave_offsets(wcnt, cnt);
+        wave_offsets<RT>(wcnt, cnt);
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < RI; ++j) {
@@ -1257,6 +1260,27 @@ void sort_stages(tsc_ctx* ctx, const int32_t* coords, int64_t N, Gen gen, int nb
   const int nbk = 1 << tb;
   const int64_t ntiles = (N + PTILE - 1) / PTILE;
   hipStream_t s = ctx->stream;
+  auto buckets = [&](K* k0, int32_t* v0, K* k1, int32_t* v1, const int* totals, const int* bstart,
+                     const GatherSrc<K>& gs) {
+    auto run = [&](auto threads) {
+      constexpr int RT = decltype(threads)::value;
+      bucket_sort_kernel<K, RT><<<(unsigned)nbk, RT, 0, s>>>(
+          k0, v0, k1, v1, kOut, vOut, totals, bstart, nbk, lb, cells, Z, ncol, N, cols, gs);
+    };
+    // 512 threads where buckets outgrow the registers (RTILE elements): their chunks, and LSD
+    // passes (ranges past the bitmap), take half as many rounds.  Below, most blocks are small or
+    // empty and twice the threads cost more than they give.  The largest bucket of a surface holds
+    // three to four times the mean.  us, 256 / 512 threads, map of shuffled shells:
+    //   50 k voxels, 256^3       27.6 / 31.2      1.15 M, 512^3       71.3 / 74.1
+    //   1.3 M, 512^3             86.7 / 79.6      1.5 M, 512^3       114.6 / 100.9
+    //   600 k, 2 x 512^3 (LSD)   95.8 / 95.9      1 M, 2 x 512^3     140.2 / 131.6
+    // Morton buckets are less even (gather plan): 150 k 48.5 / 49.8, 300 k 70.4 / 68.7, 600 k in
+    // 2 x 512^3 202 / 163.
+    const int64_t used = cells > 0 ? ((cells - 1) >> lb) + 1 : nbk;  // buckets of the key range
+    const bool wide = gs.ktile ? N > used * (lb > kBitmapBits ? 600 : 1150) : N > 200000;
+    if (wide) run(std::integral_constant<int, 512>());
+    else run(std::integral_constant<int, 256>());
+  };
   if (sb.kC) {  // carved for the gather pipeline
     {
       ProfScope p(ctx, names[0]);
@@ -1264,9 +1288,8 @@ void sort_stages(tsc_ctx* ctx, const int32_t* coords, int64_t N, Gen gen, int nb
           (const int4*)coords, N, gen, lb, tb, sb.kA, sb.vA, sb.counts, (int)ntiles, sb.oob_tile);
     }
     ProfScope ps(ctx, names[3]);
-    bucket_sort_kernel<K><<<(unsigned)nbk, RT, 0, s>>>(
-        sb.kB, sb.vB, sb.kC, sb.vC, kOut, vOut, nullptr, nullptr, nbk, lb, cells, Z, ncol, N,
-        cols, GatherSrc<K>{sb.kA, sb.vA, sb.counts, (int)ntiles, sb.oob_tile, status});
+    buckets(sb.kB, sb.vB, sb.kC, sb.vC, nullptr, nullptr,
+            GatherSrc<K>{sb.kA, sb.vA, sb.counts, (int)ntiles, sb.oob_tile, status});
     return;
   }
   {
@@ -1276,7 +1299,7 @@ void sort_stages(tsc_ctx* ctx, const int32_t* coords, int64_t N, Gen gen, int nb
   }
   {
     ProfScope ps(ctx, names[1]);
-    scan_kernel<<<(unsigned)nbk, RT, 0, s>>>(sb.counts, (int)ntiles, sb.totals, sb.oob_tile,
+    scan_kernel<<<(unsigned)nbk, ST, 0, s>>>(sb.counts, (int)ntiles, sb.totals, sb.oob_tile,
                                              status);
   }
   {
@@ -1286,9 +1309,8 @@ void sort_stages(tsc_ctx* ctx, const int32_t* coords, int64_t N, Gen gen, int nb
   }
   {
     ProfScope ps(ctx, names[3]);
-    bucket_sort_kernel<K><<<(unsigned)nbk, RT, 0, s>>>(
-        sb.kB, sb.vB, sb.kA, sb.vA, kOut, vOut, sb.totals, sb.bstart, nbk, lb, cells, Z, ncol, N,
-        cols, GatherSrc<K>{nullptr, nullptr, nullptr, 0, nullptr, nullptr});
+    buckets(sb.kB, sb.vB, sb.kA, sb.vA, sb.totals, sb.bstart,
+            GatherSrc<K>{nullptr, nullptr, nullptr, 0, nullptr, nullptr});
   }
 }
 
