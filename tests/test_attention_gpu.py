@@ -233,3 +233,22 @@ def test_attention_fp32_moving_maximum(pkg, dev, d, step):
         p = torch.softmax(torch.einsum("qhd,khd->hqk", q[s].double(), k[s].double()), dim=2)
         want = torch.einsum("hqk,khd->qhd", p, v[s].double())
         assert ((out[s].double() - want).norm() / want.norm()).item() <= 1e-4
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens_q,lens_kv,h", [
+    ([160], None, 3), ([161], None, 3),                   # few keys: blocks of 256 queries; of 128
+    ([2048], None, 16), ([2049], None, 16),               # 16 and 17 blocks of 128 a head on 256 CUs
+    ([700, 900, 1100, 1300], None, 12),                   # uneven sequences
+    ([1100, 1100], [700, 700], 16), ([1100, 1100], None, 16)])
+def test_query_blocks_at_dispatch_edges(pkg, dev, dtype, lens_q, lens_kv, h):
+    """D = 128, either side of each line between blocks of 256 and of 128 queries."""
+    d, lens_kv = 128, lens_kv or lens_q
+    rng = np.random.default_rng(sum(lens_q))
+    cu_q, cu_kv = np.cumsum([0] + lens_q).tolist(), np.cumsum([0] + lens_kv).tolist()
+    q, k, v = (torch.from_numpy(rng.standard_normal((n, h, d), np.float32)).to(dtype)
+               for n in (cu_q[-1], cu_kv[-1], cu_kv[-1]))
+    print(f"  attention query blocks {dtype} {lens_q} {lens_kv} H={h}", flush=True)
+    out = pkg.sparse_attention(q.to(dev), k.to(dev), v.to(dev), cu_q, cu_kv)
+    hs = [0, h - 1]  # heads are independent: two of them against the oracle
+    _check(out[:, hs], q[:, hs], k[:, hs], v[:, hs], cu_q, cu_kv, dtype)

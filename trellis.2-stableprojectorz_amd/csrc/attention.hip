@@ -629,13 +629,25 @@ int attention_launch(tsc_ctx* ctx, int32_t dtype, const void* q, const void* k, 
     return fail(TSC_ERR_UNSUPPORTED, "attention: %lld (head, sequence) pairs", (long long)hb);
   // Queries per block.  fp32: 128.  bf16 / f16: 256 (D = 64: four waves of 64, so that every K and V
   // fragment read from LDS serves two q tiles; D = 128: eight waves of 32, the accumulators of 64
-  // would leave one wave per SIMD) while that makes a block or more per CU (D = 64, whose blocks
-  // share a CU in pairs: 1.5), else four waves of 32.  24 x 64 bf16, two sequences: 2.5 k queries
-  // (400 blocks of 256) 88 us against 97; 16 x 64, four of 1.3 k (344 blocks) 40 against 34;
-  // 12 x 128, 2000 queries (96 blocks) 70 against 55, 9000 (432) 609 against 639.
+  // would leave one wave per SIMD), or four waves of 32 = 128 where too few blocks of 256 come
+  // together.  us, blocks of 256 / 128:
+  //   D = 64, whose blocks share a CU in pairs: 256 from 1.5 blocks of it per CU on.  24 heads, two
+  //     sequences of 2.5 k queries (264 blocks of 256) 52 / 46, of 4 k (408) 79 / 88.
+  //   D = 128: 128 while every one of those has a CU of its own: 12 heads, 2.5 k queries (240 blocks
+  //     of 128) 79 / 64, 3 k (288) 91 / 104; 12 heads, four sequences, 3 k queries on 900 keys each
+  //     40 / 45.  And, below one block of 256 per CU, self-attention over uneven sequences of 850
+  //     and more, whose blocks take as long as their sequence is: the shorter ones fill in.  12
+  //     heads, four of 4 k in all 63 / 56, two of 5 k 136 / 120, eight of 3 k 29 / 32.  Up to 160
+  //     keys a sequence the prologue decides, and half as many waves stage its first blocks in
+  //     twice the time: four of 500 in all 14.9 / 15.8.
   const int64_t tiles = std::min<int64_t>(B * (((int64_t)max_seqlen_q + 255) / 256),
                                           (total_q + 255) / 256 + B / 2);
-  const bool wide = tiles * H >= (D == 64 ? 384 : 256);
+  const bool each_a_cu = (((int64_t)max_seqlen_q + 127) / 128) * hb <= 256;
+  const bool uneven = total_kv == total_q && total_q >= 850 * (int64_t)B &&
+                      6 * B * (int64_t)max_seqlen_q >= 7 * total_q;
+  const bool wide = D == 64 ? tiles * H >= 384
+                            : total_kv <= 160 * (int64_t)B ||
+                                  (!each_a_cu && (tiles * H >= 256 || !uneven));
   const int bq = dtype == TSC_F32 ? kBQ : wide ? 256 : 128;
   // q tiles beyond the grid's x extent are covered by the kernels' tile loops
   const unsigned gx = (unsigned)std::min<int64_t>(
