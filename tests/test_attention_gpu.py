@@ -252,3 +252,24 @@ def test_query_blocks_at_dispatch_edges(pkg, dev, dtype, lens_q, lens_kv, h):
     out = pkg.sparse_attention(q.to(dev), k.to(dev), v.to(dev), cu_q, cu_kv)
     hs = [0, h - 1]  # heads are independent: two of them against the oracle
     _check(out[:, hs], q[:, hs], k[:, hs], v[:, hs], cu_q, cu_kv, dtype)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n", [64, 96, 200, 201, 500])
+def test_attention_fp32_large_values(pkg, dev, d, n):
+    """Values near the largest float, with one key in 32 that counts, each by 4 more than the one
+    before: the weights stay at most 1 against the running maximum, so no partial sum exceeds
+    1 / (1 - e^-4) = 1.02 values and the outputs are finite.  The 500 terms' fp32 roundings come to
+    less than 1e-5 of the largest."""
+    h, cu = 2, [0, n]
+    q = torch.zeros((n, h, d))
+    q[..., 0] = 1.0
+    k = torch.zeros((n, h, d))
+    k[:, :, 0] = -100.0
+    at = torch.arange(31, n, 32)
+    k[at, :, 0] = 4.0 * torch.arange(len(at), dtype=torch.float32)[:, None]
+    v = torch.full((n, h, d), 3e38)
+    print(f"  attention fp32 large values D={d} n={n}", flush=True)
+    out = pkg.sparse_attention(q.to(dev), k.to(dev), v.to(dev), cu, scale=1.0).cpu()
+    assert bool(out.isfinite().all())
+    assert ((out.double() - 3e38).abs().max() / 3e38).item() <= 1e-5

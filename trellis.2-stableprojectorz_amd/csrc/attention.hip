@@ -568,13 +568,14 @@ __global__ void __launch_bounds__(kThreads, 2)
         if (decltype(masked)::value && kb + 8 * (j >> 2) + 4 * hf + (j & 3) >= kv_len)
           s[j] = -INFINITY;
       }
-      // The maximum is raised, and what was summed rescaled, only when a score exceeds it by more
-      // than 2^kLazy for some query of the wave.
+      // What was summed is rescaled only when the maximum of some query of the wave moves.  No
+      // headroom as in the 16-bit kernels: a probability stays at most 1, or large values of v
+      // (past 2^120) would make a sum infinite that is not.
       float mx = s[0];
 #pragma unroll
       for (int j = 1; j < 16; ++j) mx = fmaxf(mx, s[j]);
       mx = pair_max(mx);
-      if (__builtin_amdgcn_ballot_w64(mx * scale_log2 > mc + kLazy) != 0) {
+      if (__builtin_amdgcn_ballot_w64(mx > m_run) != 0) {
         const float m_new = fmaxf(m_run, mx);
         const float alpha = fast_exp2((m_run - m_new) * scale_log2);  // 0 while m_run = -inf
         m_run = m_new;
