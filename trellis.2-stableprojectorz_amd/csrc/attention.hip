@@ -467,12 +467,13 @@ __global__ void __launch_bounds__(64 * NW, 2)
 }
 
 // ---------------------------------------------------------------------------------- f32
-// Two waves per SIMD, at D = 128 for a few spilled registers: one wave's softmax then runs beside the
-// other's MFMAs.  5.8 k and 9.3 k tokens, 12 x 128: 6.26 ms (118 TFLOP/s of the 154 that a large
-// fp32 product reaches; 6.92 with one wave, 7.47 with it and a rescale and the mask in every
-// block).
-template <int D>
-__global__ void __launch_bounds__(kThreads, 2)
+// W waves per SIMD.  Two, at D = 128 for 44 spilled registers (180 bytes a lane): one wave's softmax
+// then runs beside the other's MFMAs.  5.8 k and 9.3 k tokens, 12 x 128: 6.26 ms (118 TFLOP/s of
+// the 154 that a large fp32 product reaches; 6.92 with one wave, 7.47 with it and a rescale and the
+// mask in every block).  With a few blocks of keys the spills show and D = 128 takes one: 12 heads,
+// two sequences of 50 tokens 17.5 us against 19.5, of 200 48.2 against 48.3.
+template <int D, int W>
+__global__ void __launch_bounds__(kThreads, W)
     attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
                     const float* __restrict__ v, const int32_t* __restrict__ cu_q,
                     const int32_t* __restrict__ cu_kv, int64_t total_q, int64_t total_kv,
@@ -661,13 +662,13 @@ int attention_launch(tsc_ctx* ctx, int32_t dtype, const void* q, const void* k, 
         (const decltype(t)*)q, (const decltype(t)*)k, (const decltype(t)*)v, cu_q, cu_kv, total_q,
         total_kv, H, sl2, (decltype(t)*)out);
   };
+  constexpr std::integral_constant<int, 1> I1{};
+  constexpr std::integral_constant<int, 2> I2{};
+  constexpr std::integral_constant<int, 4> I4{};
+  constexpr std::integral_constant<int, 8> I8{};
+  constexpr std::integral_constant<int, 64> D64{};
+  constexpr std::integral_constant<int, 128> D128{};
   auto by_size = [&](auto t) {
-    constexpr std::integral_constant<int, 1> I1{};
-    constexpr std::integral_constant<int, 2> I2{};
-    constexpr std::integral_constant<int, 4> I4{};
-    constexpr std::integral_constant<int, 8> I8{};
-    constexpr std::integral_constant<int, 64> D64{};
-    constexpr std::integral_constant<int, 128> D128{};
     if (D == 64) wide ? mma(t, D64, I2, I4) : mma(t, D64, I1, I4);
     else wide ? mma(t, D128, I1, I8) : mma(t, D128, I1, I4);
   };
@@ -675,14 +676,15 @@ int attention_launch(tsc_ctx* ctx, int32_t dtype, const void* q, const void* k, 
     by_size(__bf16());
   } else if (dtype == TSC_F16) {
     by_size(_Float16());
-  } else if (D == 64) {
-    attn_f32_kernel<64><<<grid, kThreads, 0, ctx->stream>>>(
-        (const float*)q, (const float*)k, (const float*)v, cu_q, cu_kv, total_q, total_kv, H, sl2,
-        (float*)out);
   } else {
-    attn_f32_kernel<128><<<grid, kThreads, 0, ctx->stream>>>(
-        (const float*)q, (const float*)k, (const float*)v, cu_q, cu_kv, total_q, total_kv, H, sl2,
-        (float*)out);
+    auto f32 = [&](auto d, auto w) {
+      attn_f32_kernel<decltype(d)::value, decltype(w)::value><<<grid, kThreads, 0, ctx->stream>>>(
+          (const float*)q, (const float*)k, (const float*)v, cu_q, cu_kv, total_q, total_kv, H,
+          sl2, (float*)out);
+    };
+    if (D == 64) f32(D64, I2);
+    else if (total_kv <= 200 * (int64_t)B) f32(D128, I1);
+    else f32(D128, I2);
   }
   return check_hip(hipGetLastError(), "attention launch");
 }
