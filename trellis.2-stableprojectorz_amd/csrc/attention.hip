@@ -471,7 +471,7 @@ __global__ void __launch_bounds__(64 * NW, 2)
 // then runs beside the other's MFMAs.  5.8 k and 9.3 k tokens, 12 x 128: 6.26 ms (118 TFLOP/s of
 // the 154 that a large fp32 product reaches; 6.92 with one wave, 7.47 with it and a rescale and the
 // mask in every block).  With a few blocks of keys the spills show and D = 128 takes one: 12 heads,
-// two sequences of 50 tokens 17.5 us against 19.5, of 200 48.2 against 48.3.
+// two sequences of 50 tokens 17.1 us against 19.5, 700 queries on 300 keys each 58.2 against 60.8.
 template <int D, int W>
 __global__ void __launch_bounds__(kThreads, W)
     attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
@@ -683,7 +683,7 @@ int attention_launch(tsc_ctx* ctx, int32_t dtype, const void* q, const void* k, 
           sl2, (float*)out);
     };
     if (D == 64) f32(D64, I2);
-    else if (total_kv <= 200 * (int64_t)B) f32(D128, I1);
+    else if (total_kv <= 320 * (int64_t)B) f32(D128, I1);
     else f32(D128, I2);
   }
   return check_hip(hipGetLastError(), "attention launch");
