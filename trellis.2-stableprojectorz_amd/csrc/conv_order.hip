@@ -337,10 +337,10 @@ __device__ __forceinline__ int gr_digit(const int32_t* head, int e) {
   return 255 - (rows < 255 ? rows : 255);
 }
 
-template <int CHUNK, int T>
-__global__ void __launch_bounds__(T)
+__global__ void __launch_bounds__(kGrThreads)
     ord_greedy_kernel(const uint32_t* __restrict__ keys, const int32_t* __restrict__ vals,
                       int64_t n, int32_t* __restrict__ order) {
+  constexpr int CHUNK = kGrChunk, T = kGrThreads;
   constexpr int P = CHUNK / T;  // rows, and entries at most, per thread
   static_assert(CHUNK % kGrTile == 0, "chunks hold whole tiles");
   static_assert(CHUNK <= (1 << 14), "14-bit entry indices in the growth candidates");
@@ -587,8 +587,8 @@ int conv_order_launch(tsc_ctx* ctx, const int32_t* nbr, const int32_t* perm, int
     std::swap(kc, kn);
     std::swap(vc, vn);
   }
-  ord_greedy_kernel<kGrChunk, kGrThreads>
-      <<<(unsigned)((N + kGrChunk - 1) / kGrChunk), kGrThreads, 0, s>>>(kc, vc, N, order);
+  ord_greedy_kernel<<<(unsigned)((N + kGrChunk - 1) / kGrChunk), kGrThreads, 0, s>>>(kc, vc, N,
+                                                                                     order);
   return check_hip(hipGetLastError(), "conv_order launch");
 }
 
