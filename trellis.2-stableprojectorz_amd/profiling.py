@@ -51,7 +51,27 @@ def _conv_name(kind: str, t: str, nums: list) -> str:
     return f"conv_regstage_kernel<{t},{bm}x{bn},k{kb}{',res' if epi == '1' else ''}>"
 
 
+def _generic_name(t: str, args: list) -> str:  # LW, EPI, SPLIT, AHEAD
+    lw, epi, split, _ = args
+    return (f"conv_generic_kernel<{t},p{lw}{',split' if split in ('1', 'true') else ''}"
+            f"{',res' if epi == '1' else ''}>")
+
+
+def _split_name(args: list) -> str:  # FN (blocks of 32 columns), EPI
+    return f"conv_split_kernel<128x{32 * int(args[0])}{',res' if args[1] == '1' else ''}>"
+
+
 def short_name(name: str) -> str:
+    m = re.search(r"conv_generic_kernelI(DF16b|DF16_|f)((?:L[ib]\d+E)+)", name)  # mangled
+    if m:
+        return _generic_name(_TYPES[m.group(1)], re.findall(r"L[ib](\d+)E", m.group(2)))
+    m = re.search(r"conv_generic_kernel<(__bf16|_Float16|float), ([^>]+)>", name)  # demangled
+    if m:
+        return _generic_name(_DEMANGLED_TYPES[m.group(1)], [x.strip() for x in m.group(2).split(",")])
+    m = (re.search(r"conv_split_kernelI((?:Li\d+E)+)", name)
+         or re.search(r"conv_split_kernel<([\d, ]+)>", name))
+    if m:
+        return _split_name(re.findall(r"\d+", m.group(1)))
     kinds = "conv_mfma_kernel|conv_regstage_kernel|conv_narrow_kernel|conv_gather_kernel"
     m = re.search(rf"({kinds})I(DF16b|DF16_|f)((?:Li\d+E)+)", name)  # mangled
     if m:
