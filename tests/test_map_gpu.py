@@ -128,11 +128,11 @@ def test_map_near_sorted_input(pkg, dev, order):
     _check(m, coords, 1, (512, 512, 512), (1, 1, 1))
 
 
-@pytest.mark.parametrize("n,batch", [(1177600, 1), (1177601, 1), (614400, 2), (614401, 2)])
+@pytest.mark.parametrize("n,batch", [(716800, 1), (716801, 1), (300000, 2)])
 @pytest.mark.parametrize("shuffle", [False, True])
 def test_map_bucket_block_sizes(pkg, dev, n, batch, shuffle):
-    """Either side of the sizes at which the bucket blocks grow, for bucket ranges inside the LDS bitmap
-    (one sample) and past it (two): buckets of a few hundred voxels, one of 4096 and some of
+    """Either side of the size at which the bucket blocks grow, and a bucket range past the LDS bitmap
+    (two samples): buckets of a few hundred voxels, one of 4096 and some of
     30000.  Every output equals the bitmap build's (which the other tests hold to the oracle)."""
     cells = batch << 27
     third = n // 3

@@ -466,8 +466,11 @@ struct GatherSrc {
   uint32_t* status;
 };
 
+// RT threads per block; 512 with 32-bit keys are held to 64 registers, so that four blocks share a
+// CU: with 69, three did, and the last 256 of the 1024 blocks came in a second round (map of 1.5 M
+// voxels in even buckets: 88.8 us, now 86.2; 256 threads 86.8).
 template <typename K, int RT>
-__global__ void __launch_bounds__(RT)
+__global__ void __launch_bounds__(RT, RT == 512 && sizeof(K) == 4 ? 8 : 1)
     bucket_sort_kernel(K* k0, int32_t* v0, K* k1, int32_t* v1, K* __restrict__ kout,
                        int32_t* __restrict__ vout, const int* __restrict__ totals,
                        const int* __restrict__ bstart, int nbk,
@@ -1267,17 +1270,16 @@ void sort_stages(tsc_ctx* ctx, const int32_t* coords, int64_t N, Gen gen, int nb
       bucket_sort_kernel<K, RT><<<(unsigned)nbk, RT, 0, s>>>(
           k0, v0, k1, v1, kOut, vOut, totals, bstart, nbk, lb, cells, Z, ncol, N, cols, gs);
     };
-    // 512 threads where buckets outgrow the registers (RTILE elements): their chunks, and LSD
-    // passes (ranges past the bitmap), take half as many rounds.  Below, most blocks are small or
-    // empty and twice the threads cost more than they give.  The largest bucket of a surface holds
-    // three to four times the mean.  us, 256 / 512 threads, map of shuffled shells:
-    //   50 k voxels, 256^3       27.6 / 31.2      1.15 M, 512^3       71.3 / 74.1
-    //   1.3 M, 512^3             86.7 / 79.6      1.5 M, 512^3       114.6 / 100.9
-    //   600 k, 2 x 512^3 (LSD)   95.8 / 95.9      1 M, 2 x 512^3     140.2 / 131.6
-    // Morton buckets are less even (gather plan): 150 k 48.5 / 49.8, 300 k 70.4 / 68.7, 600 k in
-    // 2 x 512^3 202 / 163.
+    // 512 threads where the blocks have work for them: buckets past the registers (RTILE elements)
+    // or past the bitmap's range (LSD passes), whose chunks take half as many rounds.  Maps of small
+    // buckets, most of them nearly empty, run 256.  us, 256 / 512 threads, shuffled shells:
+    //   map     50 k voxels, 128^3 x 3  27.3 / 28.7     300 k, 512^3   43.3 / 44.3
+    //           700 k, 512^3  59.8 / 60.0               1 M   71.9 / 71.5     1.5 M  115.0 / 101.7
+    //     (LSD) 50 k, 2 x 512^3  52.0 / 45.8            1 M, 2 x 512^3  139.6 / 118.7
+    //   plan    50 k, 128^3 x 3  43.3 / 43.6            300 k, 512^3   70.3 / 67.3
+    //     (LSD) 50 k, 2 x 512^3  69.9 / 60.0
     const int64_t used = cells > 0 ? ((cells - 1) >> lb) + 1 : nbk;  // buckets of the key range
-    const bool wide = gs.ktile ? N > used * (lb > kBitmapBits ? 600 : 1150) : N > 200000;
+    const bool wide = !gs.ktile || lb > kBitmapBits || N > 700 * used;
     if (wide) run(std::integral_constant<int, 512>());
     else run(std::integral_constant<int, 256>());
   };
