@@ -662,3 +662,36 @@ def test_conv_fp32_from_two_threads(pkg, dev):
     for t in threads:
         t.join()
     assert not wrong
+
+
+def test_conv_fp32_captured_on_a_fresh_context(pkg, dev):
+    """The first fp32 conv of a context can be captured into a graph (an allocation or a wait would
+    fail the capture); every replay, with other convs in between, gives the eager call's bits."""
+    n, c = 3000, 64
+    nbr = torch.from_numpy(_random_table(n, 3)).to(dev)
+    f = torch.from_numpy(pkg.workloads.features(n, c, 1)).to(dev)
+    w = torch.from_numpy(pkg.workloads.conv_weight(c, c, 2)).to(dev)
+    other = torch.from_numpy(pkg.workloads.conv_weight(c, c, 3)).to(dev)
+    want = pkg.sparse_conv3d(f, w, None, nbr)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream(dev)
+    with torch.cuda.stream(side):
+        fresh = pkg._lib.Context(dev.index)
+    out = torch.empty_like(want)
+    graph = torch.cuda.CUDAGraph()
+    print("  conv fp32 captured", flush=True)
+    with torch.cuda.graph(graph, stream=side):
+        st = fresh.lib.tsc_conv(fresh.bind(), pkg._lib.TSC_F32, f.data_ptr(), w.data_ptr(), None,
+                                nbr.data_ptr(), None, n, c, c, out.data_ptr())
+    assert st == 0, fresh.lib.tsc_last_error().decode()
+    try:
+        for _ in range(3):
+            out.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+            pkg.sparse_conv3d(f, other, None, nbr)
+            torch.cuda.synchronize()
+    finally:
+        del graph
+        fresh.lib.tsc_ctx_destroy(fresh.handle)
