@@ -5,7 +5,9 @@
  * (a TS host passes them as u64 / Deno "pointer"; a Python host passes tensor.data_ptr()).
  * Every call returns an int status (TSC_OK == 0); on failure tsc_last_error() holds a message
  * for the calling thread.  All compute calls are enqueue-only on the context's stream and
- * return before the GPU finishes; tsc_sync() waits.
+ * return before the GPU finishes; tsc_sync() waits.  (Exceptions, named where they are: a context's
+ * workspaces grow with a stream synchronization, tsc_linear tunes a new shape, the subdivision
+ * counts are returned to the host.)
  *
  * Interfaces replaced (reference = johnandersen777/TRELLIS.2-stableprojectorz):
  *   SparseConv3d.forward pass0+pass1 (neighbor map)   src/sparse/ops/conv3d.ts:62-152,
@@ -159,7 +161,15 @@ int tsc_map_gather_plan(tsc_ctx* ctx, const int32_t* coords, const int32_t* nbr,
  *   Any Ci >= 1 (Ci * element size <= 65536 bytes) and 1 <= Co <= 65536, as the reference's
  *   bounds-checked shader (conv3d_wgsl.ts:174-196).  The tuned kernels run when Ci * element size
  *   is a multiple of 32 bytes, Co a multiple of 32 and every buffer 16-byte aligned; other
- *   shapes run a generic kernel (zero-padded K tail, masked Co tail), with the same arithmetic.
+ *   shapes run a generic kernel (zero-padded K tail, masked Co tail).  Alignment does not change
+ *   a result.
+ *   fp32 with Ci a multiple of 16 from 32 on and Co a multiple of 32 (not 32 -> 32) is multiplied on
+ *   the bf16 matrix cores: three bf16 pieces per value (24 bits), the six largest of their nine
+ *   products, summed in fp32.  Against fp64 a sum of many products is nearer than on fp32 matrix
+ *   cores (0.8-0.9 of the error, N(0,1) rows); a sum that is one product only is within 2.5e-7 of
+ *   it (6e-8 there).  Sums that the pieces do not hold for (infinities and NaN, operands below
+ *   2^-100 where they count) are made again on fp32 matrix cores; inputs that are below 2^-100
+ *   throughout take about three times as long for it.
  * Replaces conv3d.ts:154-221 / conv3d_wgsl.ts:132-231. */
 int tsc_conv(tsc_ctx* ctx, int32_t dtype, const void* feats, const void* weight, const void* bias,
              const int32_t* nbr, const int32_t* order, int64_t N, int32_t Ci, int32_t Co, void* out);

@@ -130,7 +130,11 @@ def check(status: int) -> None:
 
 
 class Context:
-    """One tsc_ctx per device, following torch's current stream on that device."""
+    """One tsc_ctx per device, following torch's current stream on that device.
+
+    All threads share it.  Calls that use its workspaces (map, row order, gather plan, ResBlock,
+    masked subdivision, linear, 16-bit convs on 256-row tiles) or come from different streams have
+    to be made one at a time, as the C library asks; other convs and attention keep nothing in it."""
 
     def __init__(self, device: int):
         import torch

@@ -19,10 +19,10 @@
 //   f32:      v_mfma_f32_32x32x2f32 (k-step = 2 dims / 2 keys; K and V row-major in LDS with
 //             padded strides, no transpose needed), 32-key blocks.
 // Bound: MFMA (4 * D flops per query-key pair) and the softmax's exp per pair.  Two sequences of
-// 24.7 k and 39.6 k tokens, 12 x 128 bf16: 12.8-13.6 ms (980-1040 TFLOP/s; 14.2 with one wave's
-// MFMAs and softmax in turn and V transposed on its way into LDS), MFMA busy 48 % at the 1.97 GHz
-// that the chip holds (hipBLASLt's 8192^3 bf16 product: 1.11 PFLOP/s); 20 k tokens, 24 x 64 f16:
-// 2.95 ms against 3.57; cross, 36 k queries x 1.3 k keys, 16 x 64 f16: 289 us against 365.
+// 24.7 k and 39.6 k tokens, 12 x 128 bf16: 12.9-13.3 ms (1010-1040 TFLOP/s; 14.2 with one wave's
+// MFMAs and softmax in turn and V transposed on its way into LDS), MFMA busy 49 % at 2.04 GHz
+// (hipBLASLt's 8192^3 bf16 product: 1.32 PFLOP/s); 20 k tokens, 24 x 64 f16: 2.95 ms against 3.57;
+// cross, 36 k queries x 1.3 k keys, 16 x 64 f16: 268 us against 365.
 
 #include <type_traits>
 
@@ -102,8 +102,8 @@ __device__ __forceinline__ void segment(const int32_t* cu, int b, int64_t total,
 // round robin.  Every XCD gets the same share of every sequence, whatever the sequences' lengths:
 // of each eight heads XCD x takes one, so that a head's K and V come into one L2 only, and the q
 // tiles of the heads past a multiple of eight are spread over all XCDs.  (Contiguous runs of
-// blocks per XCD left the XCDs of the short sequences idle: 20.4 ms against 14.7 ms for sequences
-// of 24.7 k and 39.6 k tokens, 12 x 128 bf16.)
+// blocks per XCD left the XCDs of the short sequences idle: 21.1 ms against 14.2 ms for sequences
+// of 24.7 k and 39.6 k tokens, 12 x 128 bf16, MFMAs and softmax still in turn.)
 // Sequences with more keys go first, so that the launch ends on its shortest blocks; past
 // kMaxRanked sequences the ranking would cost more than the tail it saves, and they keep their
 // order.

@@ -16,7 +16,7 @@
 //   conv_mfma_kernel      rows longer than 64 bytes (wide channels, several chunks per tap):
 //                         a 3-8 stage ring filled by direct-to-LDS loads (global_load_lds),
 //                         per-tap source addresses kept in registers, fragments read with
-//                         explicit LDS waits, one block of 4 waves per CU
+//                         explicit LDS waits
 //   conv_regstage_kernel  rows of at most 64 bytes (one chunk per tap): register-staged double
 //                         buffer, one barrier per chunk, two blocks per CU
 //
@@ -1394,11 +1394,12 @@ __device__ __forceinline__ int swz_split(int row, int part) { return part ^ ((ro
 // and MFMAs overlap.  Loads are unconditional (past the end: the last weights again, zero
 // rows): with branches around them the compiler waits for every load in flight before the first use
 // of a row.
-// Bound: the bf16 matrix rate at what the chip's power allows, with 12-67 % more taps than the rows
-// have.  us, fp32 MFMA ring kernel / weights split beforehand in device memory / this: 32->64 on
-// 1.5 M voxels 788 / 597 / 560, 64->64 on 300 k 478 / 330 / 303, 512->512 on 10 k
-// 1519 / 921 / 820.  Looking for small weights is 1-2 % of that (for small inputs too, in every
-// chunk: 5-16 %).
+// Bound: vector instructions (128 x 64 columns: 100 beside the 12 MFMAs of a wave's chunk, 66 of them
+// splits) and one barrier per chunk; matrix cores busy 29 % at 2.1 GHz on 32->64 at 1.5 M voxels,
+// where a tile's taps are 1.5x the valid ones.  us, fp32 MFMA ring kernel / weights split beforehand
+// in device memory / this: 32->64 on 1.5 M voxels 788 / 597 / 560, 64->64 on 300 k 478 / 330 / 303,
+// 512->512 on 10 k 1519 / 921 / 820.  Looking for small weights is 1-2 % of that (for small inputs
+// too, in every chunk: 5-16 %).
 constexpr int kSplitBM = 128, kSplitThreads = 256;
 template <int FN, int EPI>
 __global__ void __launch_bounds__(kSplitThreads, FN == 2 ? 4 : 1)

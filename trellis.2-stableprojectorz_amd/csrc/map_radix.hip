@@ -559,7 +559,7 @@ __global__ void __launch_bounds__(RT, RT == 512 && sizeof(K) == 4 ? 8 : 1)
         // A run longer than kLongRun is expanded by its whole wave, 64 positions at a time: where
         // the input is close to sorted (the children of a subdivision) a bucket is one or two runs
         // of thousands, which one thread walked alone (map of 1.4 M children in 512^3, this
-        // kernel: 164 us, now 30).  Shuffled input has runs of ~8, one thread each.
+        // kernel: 164 us, now 25).  Shuffled input has runs of ~8, one thread each.
         const int lo = max(rb0[k], c0), hi = min(rb0[k] + rl[k], c1);  // empty: lo >= hi
         const int src = (k * RT + tid) * PTILE + ra[k] - rb0[k];
         const bool longrun = hi - lo > kLongRun;

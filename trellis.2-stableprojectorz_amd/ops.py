@@ -197,7 +197,8 @@ def sparse_conv3d(feats: torch.Tensor, weight: torch.Tensor, bias, nmap, order=N
 
     weight is (Co,Kd,Kh,Kw,Ci) = (Co,3,3,3,Ci), same dtype as feats; accumulation is fp32.
     nmap is a NeighborMap (its cached row order, or for Ci = 32 in fp16/bf16 its cached gather
-    plan, or for small convs of the generic kernel its key order, is used for locality) or an (N,27) int32 table.
+    plan, or for small convs of the generic kernel its key order, is used for locality) or an
+    (N,27) int32 table.
     """
     plan = nmap.gather_plan() if _uses_gather_plan(nmap, order, feats, weight) else None
     key_order = (feats.dim() == 2 and weight.dim() == 5 and
