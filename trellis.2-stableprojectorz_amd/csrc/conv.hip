@@ -1623,7 +1623,7 @@ constexpr int kGenBM = 64, kGenBN = 64, kGenThreads = 256;
 // SPLIT: shapes of conv_split_kernel in buffers that are not 16-byte aligned: its arithmetic, in its
 // chunks of 64 bytes, so that alignment does not change a result.
 template <typename T, int LW, int EPI, bool SPLIT, int AHEAD>
-__global__ void __launch_bounds__(kGenThreads)
+__global__ void __launch_bounds__(kGenThreads, SPLIT ? 5 : 1)
     conv_generic_kernel(const T* __restrict__ feats, const T* __restrict__ weight,
                         const T* __restrict__ bias, const int32_t* __restrict__ nbr,
                         const int32_t* __restrict__ order, int64_t N, int32_t Ci, int32_t Co,
@@ -1698,9 +1698,9 @@ __global__ void __launch_bounds__(kGenThreads)
       };
       split_row(sA[buf], ar, as);
       split_row(sB[buf], br, bs[0]);
+      split_mma<1>(as, bs, *(f32x16_t(*)[1])&acc);
 #pragma unroll
       for (int i = 0; i < 8; i += 2) range.add(x[i], x[i + 1]);
-      split_mma<1>(as, bs, *(f32x16_t(*)[1])&acc);
     } else {
       const uint4 a = *(const uint4*)(&sA[buf][ar * KB + swz<2>(ar, part) * 16]);
       const uint4 b = *(const uint4*)(&sB[buf][br * KB + swz<2>(br, part) * 16]);
