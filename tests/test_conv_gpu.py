@@ -566,7 +566,7 @@ def test_conv_generic_by_grid_size(pkg, dev, dtype, ci, co, n):
 
 
 @pytest.mark.parametrize("sx,sw", [(1e-36, 1.0), (1e-37, 1.0), (1e-39, 1e10), (1.0, 1e-36),
-                                   (1e10, 1e-39), (1e-20, 1e-16)])
+                                   (1e10, 1e-39), (1e-20, 1e-16), (0.0, 1.0), (0.0, 1e-36)])
 @pytest.mark.parametrize("n,ci,co,misaligned", [(300, 32, 64, False), (33000, 48, 64, False),
                                                 (300, 64, 96, True)])
 def test_conv_fp32_split_small_values(pkg, dev, n, ci, co, misaligned, sx, sw):

@@ -1301,12 +1301,28 @@ __device__ __forceinline__ void split_redo(const float* feats, const float* w,
     if (acc[e] * 0.f != 0.f || !(fabsf(acc[e]) >= err[e] * 0x1p-106f)) acc[e] = sum[e];
 }
 
+// Bits of a thread's row inputs: zero if all of them are (but for a sign).  asm: as in SplitRange.
+struct SplitBits {
+  uint32_t any = 0u;
+  __device__ __forceinline__ void add(const float (&x)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; i += 2)
+      asm volatile("v_or3_b32 %0, %0, %1, %2" : "+v"(any) : "v"(x[i]), "v"(x[i + 1]));
+  }
+  // Bit r: row r of the wave has an input that is not zero.
+  __device__ __forceinline__ uint32_t rows() const {
+    const uint64_t m = __ballot(any << 1 != 0u);
+    return (uint32_t)(m | m >> 32);
+  }
+};
+
 // After the sums: makes those again that the split does not hold for.  live: bit r: row r of the
-// wave exists; hiw: the largest |weight| of this lane's columns; wsmall (uniform): the wave has used
-// a small weight.  A sum can only be too small for its small inputs if it is below 27 Ci hiw 2^-106
-// (c doubles that twice, for the roundings of E and of this): for weights of ordinary size only
-// a sum of zero is, and only then, or after a small weight, the wave looks at its inputs (64->64 on
-// 25 k voxels: 59 us, all inputs zero 97, all of 1e-36 217; the fp32 MFMA kernel took 73).
+// wave has inputs (the sums of one that has none are zero, and right); hiw: the largest |weight| of
+// this lane's columns; wsmall (uniform): the wave has used a small weight.  A sum can only be too
+// small for its small inputs if it is below 27 Ci hiw 2^-106 (c doubles that twice, for the roundings
+// of E and of this): for weights of ordinary size only a sum of zero is, and only then, or after a
+// small weight, the wave looks at its inputs (64->64 on 25 k voxels: 59 us, with a zero sum in every
+// wave 97, all inputs of 1e-36 217; the fp32 MFMA kernel took 73).
 template <int FN>
 __device__ __forceinline__ void split_finish(const float* feats, const float* w,
                                              const int32_t* nbr27, uint32_t taps, int32_t Ci,
@@ -1327,7 +1343,7 @@ __device__ __forceinline__ void split_finish(const float* feats, const float* w,
     look |= least[j] < c * hiw[j];
   }
   redo = z != 0.f;
-  if (__any(look) && live != ~0u) {  // without the rows that are not there
+  if (__any(look) && live != ~0u) {  // without the rows that have none
     look = wsmall;
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
@@ -1398,8 +1414,8 @@ __device__ __forceinline__ int swz_split(int row, int part) { return part ^ ((ro
 // splits) and one barrier per chunk; matrix cores busy 29 % at 2.1 GHz on 32->64 at 1.5 M voxels,
 // where a tile's taps are 1.5x the valid ones.  us, fp32 MFMA ring kernel / weights split beforehand
 // in device memory / this: 32->64 on 1.5 M voxels 788 / 597 / 560, 64->64 on 300 k 478 / 330 / 303,
-// 512->512 on 10 k 1519 / 921 / 820.  Looking for small weights is 1-2 % of that (for small inputs
-// too, in every chunk: 5-16 %).
+// 512->512 on 10 k 1519 / 921 / 820.  Looking for small weights and for rows without inputs is
+// 2-3 % of that (for small inputs, in every chunk: 5-16 %).
 constexpr int kSplitBM = 128, kSplitThreads = 256;
 template <int FN, int EPI>
 __global__ void __launch_bounds__(kSplitThreads, FN == 2 ? 4 : 1)
@@ -1506,6 +1522,7 @@ __global__ void __launch_bounds__(kSplitThreads, FN == 2 ? 4 : 1)
     }
   };
 
+  SplitBits bits;
   float x[AHEAD][8], w[AHEAD][WF];
   auto step = [&](int i) {
     // After the barrier every wave's part of this chunk is in LDS, and every wave has read the
@@ -1523,6 +1540,7 @@ __global__ void __launch_bounds__(kSplitThreads, FN == 2 ? 4 : 1)
       }
     uint4 as[3];
     split8(x[i], as);
+    bits.add(x[i]);
     load_a(x[i]);
     split_mma<FN>(as, bs, acc);
     const int n = (i + 1) % AHEAD;
@@ -1553,8 +1571,7 @@ __global__ void __launch_bounds__(kSplitThreads, FN == 2 ? 4 : 1)
 #pragma unroll
   for (int j = 0; j < FN; ++j) hiw[j] = __uint_as_float(sHi[32 * j + l32]);
   split_finish<FN>(feats, weight + (int64_t)col * kTaps * Ci, sNbr + myrow * kTaps, mask, Ci,
-                   (uint32_t)__ballot(sRow[myrow] >= 0), hiw,
-                   __builtin_amdgcn_readfirstlane(sSmall) != 0u, acc);
+                   bits.rows(), hiw, __builtin_amdgcn_readfirstlane(sSmall) != 0u, acc);
 
   // A store writes 32 consecutive columns of two rows.  Residual values first: all loads before
   // the first store (an output may alias the residual element by element).
@@ -1686,6 +1703,7 @@ __global__ void __launch_bounds__(kGenThreads, SPLIT ? 5 : 1)
   const int part = lane >> 5;
   const int ar = wm * 32 + (lane & 31), br = wn * 32 + (lane & 31);
   SplitRange range;  // of this lane's column's weights
+  SplitBits bits;    // of its row's inputs
   auto compute = [&](int buf) {
     if constexpr (SPLIT) {
       uint4 as[3], bs[1][3];
@@ -1697,6 +1715,7 @@ __global__ void __launch_bounds__(kGenThreads, SPLIT ? 5 : 1)
         split8(x, o);
       };
       split_row(sA[buf], ar, as);
+      bits.add(x);
       split_row(sB[buf], br, bs[0]);
       split_mma<1>(as, bs, *(f32x16_t(*)[1])&acc);
 #pragma unroll
@@ -1834,8 +1853,8 @@ __global__ void __launch_bounds__(kGenThreads, SPLIT ? 5 : 1)
   if constexpr (SPLIT) {
     const float hiw[1] = {fmaxf(range.hi, __shfl_xor(range.hi, 32, 64))};
     split_finish<1>((const float*)feats, (const float*)weight + (int64_t)co * kTaps * Ci,
-                    sNbr + ar * kTaps, mask, Ci, (uint32_t)__ballot(sRow[ar] >= 0), hiw,
-                    __any(range.small()), *(f32x16_t(*)[1])&acc);
+                    sNbr + ar * kTaps, mask, Ci, bits.rows(), hiw, __any(range.small()),
+                    *(f32x16_t(*)[1])&acc);
   }
   const float bv = bias ? to_f32<T>(bias[co]) : 0.f;
   // Residual values first, all loads before the first store (see conv_regstage_kernel).
