@@ -235,6 +235,26 @@ def test_attention_fp32_moving_maximum(pkg, dev, d, step):
         assert ((out[s].double() - want).norm() / want.norm()).item() <= 1e-4
 
 
+@pytest.mark.parametrize("lens_q,lens_kv,h", [
+    ([40, 300], [70, 90], 16), ([128] * 4, [81, 80, 82, 78], 65),  # 80 keys a sequence; 81
+    ([1025, 900], [512, 512], 14), ([1025, 900], [512, 513], 14), ([1025, 900], [512, 512], 15),
+    ([1600, 1500], [320, 320], 24), ([1600, 1500], [320, 321], 24), ([1600, 1500], [320, 320], 30)])
+def test_fp32_waves_at_dispatch_edges(pkg, dev, lens_q, lens_kv, h):
+    """fp32, D = 128, either side of each line between one and two waves per SIMD (252 and 270 blocks,
+    624 and 780).  Each head has the bits that it has alone, in a grid of its own."""
+    d = 128
+    rng = np.random.default_rng(sum(lens_q))
+    cu_q, cu_kv = np.cumsum([0] + lens_q).tolist(), np.cumsum([0] + lens_kv).tolist()
+    q, k, v = (torch.from_numpy(rng.standard_normal((n, h, d), np.float32))
+               for n in (cu_q[-1], cu_kv[-1], cu_kv[-1]))
+    print(f"  attention fp32 waves {lens_q} {lens_kv} H={h}", flush=True)
+    out = pkg.sparse_attention(q.to(dev), k.to(dev), v.to(dev), cu_q, cu_kv)
+    hs = [0, h - 1]
+    _check(out[:, hs], q[:, hs], k[:, hs], v[:, hs], cu_q, cu_kv, torch.float32)
+    q, k, v = (x[:, hs].contiguous().to(dev) for x in (q, k, v))
+    assert torch.equal(out[:, hs], pkg.sparse_attention(q, k, v, cu_q, cu_kv))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("lens_q,lens_kv,h", [
     ([160], None, 3), ([161], None, 3),                   # few keys: blocks of 256 queries; of 128

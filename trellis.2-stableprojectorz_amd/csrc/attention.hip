@@ -470,8 +470,8 @@ __global__ void __launch_bounds__(64 * NW, 2)
 // W waves per SIMD.  Two, at D = 128 for 44 spilled registers (180 bytes a lane): one wave's softmax
 // then runs beside the other's MFMAs.  5.8 k and 9.3 k tokens, 12 x 128: 6.26 ms (118 TFLOP/s of
 // the 154 that a large fp32 product reaches; 6.92 with one wave, 7.47 with it and a rescale and the
-// mask in every block).  With a few blocks of keys the spills show and D = 128 takes one: 12 heads,
-// two sequences of 50 tokens 17.1 us against 19.5, 700 queries on 300 keys each 58.2 against 60.8.
+// mask in every block).  D = 128 takes one where the spills show and the second wave does not
+// (attention_launch).
 template <int D, int W>
 __global__ void __launch_bounds__(kThreads, W)
     attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
@@ -682,9 +682,19 @@ int attention_launch(tsc_ctx* ctx, int32_t dtype, const void* q, const void* k, 
           (const float*)q, (const float*)k, (const float*)v, cu_q, cu_kv, total_q, total_kv, H,
           sl2, (float*)out);
     };
+    // D = 128, one wave per SIMD and so one block per CU, or two.  us, 12 heads, one / two:
+    //   up to 80 keys a sequence the spills are most of it: 8 x 700 queries on 64 keys 69 / 77,
+    //     5 k on 77 52.4 / 52.2;
+    //   a grid that gives no CU a second block: 2 x 700 on 258 keys 50 / 55, on 500 78 / 84; from
+    //     there on they are alike (8 x 50 on 900 165 / 170, 50 on 900 118 / 115);
+    //   one of 2.35 to 3 blocks per CU, which the pairs take two rounds for as well, on not many
+    //     keys: 8 x 700 on 258 147 / 160, on 320 184 / 200.
+    // Else two: 2 x 1.2 k on 258 106 / 98, 4 x 1.2 k on 128 84 / 61, 8 x 1.2 k on 150 153 / 125.
+    const int64_t blocks = (int64_t)gx * hb;
+    const bool one = total_kv <= 80 * (int64_t)B || (total_kv <= 512 * (int64_t)B && blocks <= 256) ||
+                     (total_kv <= 320 * (int64_t)B && blocks >= 600 && blocks <= 768);
     if (D == 64) f32(D64, I2);
-    else if (total_kv <= 320 * (int64_t)B) f32(D128, I1);
-    else f32(D128, I2);
+    else one ? f32(D128, I1) : f32(D128, I2);
   }
   return check_hip(hipGetLastError(), "attention launch");
 }
