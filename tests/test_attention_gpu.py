@@ -260,6 +260,7 @@ def test_fp32_waves_at_dispatch_edges(pkg, dev, lens_q, lens_kv, h):
     ([160], None, 3), ([161], None, 3),                   # few keys: blocks of 256 queries; of 128
     ([2048], None, 16), ([2049], None, 16),               # 16 and 17 blocks of 128 a head on 256 CUs
     ([700, 900, 1100, 1300], None, 12),                   # uneven sequences
+    ([1000, 400], None, 17), ([1000, 399], None, 17),
     ([1100, 1100], [700, 700], 16), ([1100, 1100], None, 16)])
 def test_query_blocks_at_dispatch_edges(pkg, dev, dtype, lens_q, lens_kv, h):
     """D = 128, either side of each line between blocks of 256 and of 128 queries."""

@@ -637,15 +637,16 @@ int attention_launch(tsc_ctx* ctx, int32_t dtype, const void* q, const void* k, 
   //     sequences of 2.5 k queries (264 blocks of 256) 52 / 46, of 4 k (408) 79 / 88.
   //   D = 128: 128 while every one of those has a CU of its own: 12 heads, 2.5 k queries (240 blocks
   //     of 128) 79 / 64, 3 k (288) 91 / 104; 12 heads, four sequences, 3 k queries on 900 keys each
-  //     40 / 45.  And, below one block of 256 per CU, self-attention over uneven sequences of 850
+  //     40 / 45.  And, below one block of 256 per CU, self-attention over uneven sequences of 700
   //     and more, whose blocks take as long as their sequence is: the shorter ones fill in.  12
-  //     heads, four of 4 k in all 63 / 56, two of 5 k 136 / 120, eight of 3 k 29 / 32.  Up to 160
+  //     heads, four of 4 k in all 63 / 56, two of 5 k 136 / 120, eight of 3 k 29 / 32; 8 heads,
+  //     three of 430 to 1283 47 / 38.  Up to 160
   //     keys a sequence the prologue decides, and half as many waves stage its first blocks in
   //     twice the time: four of 500 in all 14.9 / 15.8.
   const int64_t tiles = std::min<int64_t>(B * (((int64_t)max_seqlen_q + 255) / 256),
                                           (total_q + 255) / 256 + B / 2);
   const bool each_a_cu = (((int64_t)max_seqlen_q + 127) / 128) * hb <= 256;
-  const bool uneven = total_kv == total_q && total_q >= 850 * (int64_t)B &&
+  const bool uneven = total_kv == total_q && total_q >= 700 * (int64_t)B &&
                       6 * B * (int64_t)max_seqlen_q >= 7 * total_q;
   const bool wide = D == 64 ? tiles * H >= 384
                             : total_kv <= 160 * (int64_t)B ||
